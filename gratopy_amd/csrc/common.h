@@ -55,6 +55,7 @@ struct Arith<float> {
   // v_rcp_f32: 1 ulp; the projections tolerate it (reference OpenCL allows
   // 2.5 ulp for single precision division).
   static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+  static __device__ __forceinline__ float rcp_positive(float x) { return rcp(x); }
   static __device__ __forceinline__ float clamp(float x, float lo, float hi) {
     return __builtin_amdgcn_fmed3f(x, lo, hi);
   }
@@ -65,6 +66,14 @@ struct Arith<float> {
 template <>
 struct Arith<double> {
   static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+  // x positive, normal and finite: the hardware estimate and two Newton steps
+  // (to within 1 ulp, as against the correctly rounded division's 0.5), without
+  // the division's scaling and special cases
+  static __device__ __forceinline__ double rcp_positive(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+  }
   static __device__ __forceinline__ double clamp(double x, double lo, double hi) {
     return fmin(fmax(x, lo), hi);
   }

@@ -17,6 +17,7 @@
 #include <string>
 
 #include "kernels.h"
+#include "stack.h"
 
 namespace gt {
 
@@ -432,6 +433,75 @@ static void launch_back(hipStream_t st, const Job<real> &J, int nbands, int stag
   }
 }
 
+// ---- slice-batched backprojection (back_stack_tile) --------------------------
+// What bounds it: two FMAs per pixel-angle and slice (FMAs issue once per CU
+// and clock), beside them LDS reads of 32 bytes per four slices.  Summing one
+// slice at a time, as the staged kernels above do, also pays 9 instructions of
+// detector coordinate, one of them v_rcp_f32 at half rate, per pixel-angle and
+// slice; here they serve 8 slices.  32 x 2048^2, 1440 angles: fan 43.5 -> 19.2
+// ms, parallel beam 27.4 -> 15.4 ms; 16 x 512^2 fan, 360 angles: float32 446 ->
+// 211 us, float64 1150 -> 480 us.  The card then clocks at 1.97 GHz (2.2 GHz in
+// the staged kernels): it is held by power as much as by issue.
+//
+// Prologue: the padded, pre-weighted sinogram in entries of slices and the
+// angle table.  Block: 32 bins x 32 angles of one slice group; a C-ordered
+// stack (slices fastest) is read along angles and transposed through LDS so
+// that reads and writes both run along memory.
+template <typename real>
+__global__ __launch_bounds__(256) void stage_stack_kernel(Entry<real> *__restrict__ S,
+                                                          AngleRec<real> *__restrict__ tab,
+                                                          const real *__restrict__ sino, Strides3 si,
+                                                          const real *__restrict__ ofs,
+                                                          const real *__restrict__ sdpd,
+                                                          const real *__restrict__ geo, int fan, int Ns,
+                                                          int Na, int Nz) {
+  __shared__ Entry<real> tile[32][33];
+  const int Nsp = Ns + 4, q = blockIdx.z;
+  const int j0 = blockIdx.x * 32, a0 = blockIdx.y * 32;
+  const int lx = threadIdx.x & 31, ly = threadIdx.x >> 5;
+  const bool bins_first = si.s0 <= si.s1;
+  for (int k = ly; k < 32; k += 8) {
+    const int j = j0 + (bins_first ? lx : k), a = a0 + (bins_first ? k : lx);
+    if (j >= Nsp || a >= Na) continue;
+    const int s = j - 2;
+    const bool in = s >= 0 && s < Ns;
+    Entry<real> e;
+#pragma unroll
+    for (int i = 0; i < kSlices<real>; ++i) {
+      const int z = q * kSlices<real> + i;
+      e.v[i] = 0;
+      if (in && z < Nz) {
+        const real x = sino[s * si.s0 + a * si.s1 + z * si.s2];
+        e.v[i] = fan ? x * sdpd[s] * (ofs[8 * (int64_t)a + 6] / geo[0]) : x * ofs[8 * (int64_t)a + 4];
+      }
+    }
+    if (bins_first)
+      S[((int64_t)q * Na + a) * Nsp + j] = e;
+    else
+      tile[lx][k] = e;
+  }
+  if (!bins_first) {
+    __syncthreads();
+    for (int k = ly; k < 32; k += 8) {
+      const int j = j0 + lx, a = a0 + k;
+      if (j < Nsp && a < Na) S[((int64_t)q * Na + a) * Nsp + j] = tile[k][lx];
+    }
+  }
+  if (blockIdx.x == 0 && q == 0 && threadIdx.x < 32 && a0 + (int)threadIdx.x < Na)
+    back_table_entry(tab, ofs, geo, fan, a0 + (int)threadIdx.x);
+}
+
+// blockIdx.x = band + nbands * tile column, as in the staged kernels above.
+template <typename real, bool FAN, int G, int RP, int CAP, int WAVES>
+__global__ __launch_bounds__(256, WAVES) void back_stack_kernel(Job<real> J, real *part, int nbands) {
+  __shared__ StackShared<real, G, CAP> sh;
+  const int band = nbands > 1 ? blockIdx.x % nbands : 0;
+  const int bx = nbands > 1 ? blockIdx.x / nbands : blockIdx.x;
+  const int a0 = (int)((int64_t)J.Na * band / nbands);
+  const int a1 = (int)((int64_t)J.Na * (band + 1) / nbands);
+  back_stack_tile<real, FAN, G, RP, CAP>(J, bx, blockIdx.y, blockIdx.z, a0, a1, part, band, sh);
+}
+
 // ---------------------------------------------------------------------------
 // Single-line (impulse response) kernels for the sparse system matrix.
 // ---------------------------------------------------------------------------
@@ -649,6 +719,59 @@ static size_t back_ws(int dtype, const Layout &L) {
          align_up(elem_size(dtype) * (size_t)(L.Ns + 4) * L.Na * L.Nz) + back_partials(dtype, L);
 }
 
+// Slice-batched backprojection (stack.h): groups of `slices` slices per entry,
+// g groups and rp pixels per lane, angle bands.  g = 0: the launch shapes above.
+struct BackStackShape {
+  int g, rp, bands;
+  int64_t tiles(const Layout &L, int slices) const {
+    return (int64_t)((L.Nx + 31) / 32) * ((L.Ny + 8 * rp - 1) / (8 * rp)) *
+           ((L.Nz + slices * g - 1) / (slices * g));
+  }
+};
+
+static BackStackShape back_stack_shape(int dtype, const Layout &L) {
+  BackStackShape s{0, 0, 1};
+  const int slices = 16 / (int)elem_size(dtype);
+  // From half-filled entries on (two float32 slices of four leave it level
+  // with the staged kernels: 512^2 fan, 360 angles, 2 slices 83 against 79 us,
+  // 3 slices of a 700^2 fan 181 against 230 us), and for calls that are more
+  // than their launches (below 2e7 pixel-angles both take the ~31 us of the
+  // host's call).
+  if (!tuning().automatic || L.Nz == 1 || 2 * L.Nz <= slices || work_of(L) < 2e7) return s;
+  if (L.Ns >= 1 << 26) return s;  // byte offsets along a row of entries stay within int
+  // Two groups per lane (the coordinates then serve twice the slices: 32 x
+  // 2048^2 fan 19.2 ms against 21.9 with one) unless the second would be empty
+  // for more than 15 % of the slots.
+  const int fill1 = (L.Nz + slices - 1) / slices, fill2 = (fill1 + 1) / 2 * 2;
+  s.g = fill2 * 100 <= fill1 * 115 ? 2 : 1;
+  // Four pixels per lane while their tiles give every CU 6 blocks (32 x 2048^2
+  // fan: 19.2 ms against 20.5 with two), else two (16 x 512^2 fan: 211 us
+  // against 247).
+  s.rp = 4;
+  if (s.tiles(L, slices) < 1536) s.rp = 2;
+  // Angle bands up to 4 blocks per CU (9 x 301 x 257 fan, 179 angles, 510
+  // tiles: 80 / 62 / 60 us over 1 / 2 / 4 bands).
+  while (s.bands < 8 && s.tiles(L, slices) * s.bands < 1024) s.bands *= 2;
+  return s;
+}
+
+static size_t back_stack_sino(int dtype, const Layout &L, const BackStackShape &s) {
+  const size_t slices = 16 / elem_size(dtype);
+  const size_t groups = ((size_t)L.Nz + slices * s.g - 1) / (slices * s.g) * s.g;
+  return align_up((size_t)16 * groups * (size_t)(L.Ns + 4) * L.Na);
+}
+
+static size_t back_stack_ws(int dtype, const Layout &L, const BackStackShape &s) {
+  const size_t e = elem_size(dtype);
+  return align_up(e * 8 * (size_t)L.Na) + back_stack_sino(dtype, L, s) +
+         (s.bands > 1 ? align_up(e * (size_t)s.bands * L.Nx * L.Ny * L.Nz) : 0);
+}
+
+static size_t back_need(int dtype, const Layout &L) {
+  const BackStackShape s = back_stack_shape(dtype, L);
+  return s.g ? back_stack_ws(dtype, L, s) : back_ws(dtype, L);
+}
+
 template <typename real>
 static Job<real> make_job(bool fan, const Layout &L, const real *ofs, const real *sdpd,
                           const real *geo) {
@@ -806,11 +929,59 @@ static int fwd_impl(hipStream_t st, real *sino, const real *img, const real *ofs
   return check_launch(FAN ? "fan forward projection" : "radon forward projection");
 }
 
+template <typename real, bool FAN, int G, int RP, int CAP, int WAVES>
+static void launch_back_stack(hipStream_t st, const Job<real> &J, const BackStackShape &sh, real *part) {
+  constexpr int slices = kSlices<real> * G;
+  const dim3 grid((unsigned)((J.Nx + 31) / 32 * sh.bands), (J.Ny + 8 * RP - 1) / (8 * RP),
+                  (J.Nz + slices - 1) / slices);
+  hipLaunchKernelGGL((back_stack_kernel<real, FAN, G, RP, CAP, WAVES>), grid, dim3(256), 0, st, J, part,
+                     sh.bands);
+}
+
+template <typename real, bool FAN>
+static int back_stack_impl(hipStream_t st, real *img, const real *sino, const real *ofs, const real *sdpd,
+                           const real *geo, const Layout &L, int img_order, int sino_order, char *w,
+                           const BackStackShape &sh) {
+  constexpr int Q = kSlices<real>;
+  constexpr int dtype = sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32;
+  const int groups = (L.Nz + Q * sh.g - 1) / (Q * sh.g) * sh.g;
+  AngleRec<real> *tab = reinterpret_cast<AngleRec<real> *>(w);
+  w += align_up(sizeof(real) * 8 * (size_t)L.Na);
+  Entry<real> *S = reinterpret_cast<Entry<real> *>(w);
+  w += back_stack_sino(dtype, L, sh);
+  real *part = sh.bands > 1 ? reinterpret_cast<real *>(w) : nullptr;
+  hipLaunchKernelGGL(stage_stack_kernel<real>, dim3((L.Ns + 4 + 31) / 32, (L.Na + 31) / 32, groups),
+                     dim3(256), 0, st, S, tab, sino, order_strides(sino_order, L.Ns, L.Na, L.Nz), ofs, sdpd,
+                     geo, (int)FAN, L.Ns, L.Na, L.Nz);
+  Job<real> J = make_job<real>(FAN, L, ofs, sdpd, geo);
+  J.img = img;
+  J.io = order_strides(img_order, L.Nx, L.Ny, L.Nz);
+  J.S = S[0].v;
+  J.tab = tab;
+  if (sh.g == 2 && sh.rp == 4)
+    launch_back_stack<real, FAN, 2, 4, 512, 3>(st, J, sh, part);
+  else if (sh.g == 2)
+    launch_back_stack<real, FAN, 2, 2, 384, 4>(st, J, sh, part);
+  else if (sh.rp == 4)
+    launch_back_stack<real, FAN, 1, 4, 512, 5>(st, J, sh, part);
+  else
+    launch_back_stack<real, FAN, 1, 2, 384, 6>(st, J, sh, part);
+  if (part)
+    hipLaunchKernelGGL(back_reduce_kernel<real>, dim3((L.Nx + 15) / 16, (L.Ny + 15) / 16, L.Nz), dim3(256),
+                       0, st, J, part, sh.bands);
+  return check_launch(FAN ? "fan backprojection" : "radon backprojection");
+}
+
 template <typename real, bool FAN>
 static int back_impl(hipStream_t st, real *img, const real *sino, const real *ofs,
                      const real *sdpd, const real *geo, const Layout &L, int img_order,
                      int sino_order, void *ws, size_t ws_bytes) {
-  const size_t need = back_ws(sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32, L);
+  const int dtype = sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32;
+  const BackStackShape ss = back_stack_shape(dtype, L);
+  if (ss.g && ws != nullptr && ws_bytes >= back_stack_ws(dtype, L, ss))
+    return back_stack_impl<real, FAN>(st, img, sino, ofs, sdpd, geo, L, img_order, sino_order,
+                                      static_cast<char *>(ws), ss);
+  const size_t need = back_ws(dtype, L);
   if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
   GT_REQUIRE(ws != nullptr, "workspace pointer is NULL");
   char *w = static_cast<char *>(ws);
@@ -860,7 +1031,7 @@ extern "C" size_t gt_projection_workspace_bytes(int geometry, int adjoint, int d
                                                 int Ny, int Ns, int Na, int Nz, int in_order) {
   if (Nx <= 0 || Ny <= 0 || Ns <= 0 || Na <= 0 || Nz <= 0) return 0;
   const Layout L{Nx, Ny, Ns, Na, Nz, geometry == GT_GEOMETRY_FAN};
-  return adjoint ? back_ws(dtype, L) : fwd_ws(dtype, L, in_order);
+  return adjoint ? back_need(dtype, L) : fwd_ws(dtype, L, in_order);
 }
 
 extern "C" int gt_projection_shape(int geometry, int adjoint, int Nx, int Ny, int Ns, int Na,
