@@ -59,6 +59,8 @@ struct Arith<float> {
   static __device__ __forceinline__ float clamp(float x, float lo, float hi) {
     return __builtin_amdgcn_fmed3f(x, lo, hi);
   }
+  // to [0, 1], NaN to 0 (the clamp modifier of the producing instruction)
+  static __device__ __forceinline__ float clamp01(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); }
   // x - floor(x), exact (v_fract_f32)
   static __device__ __forceinline__ float fract(float x) { return __builtin_amdgcn_fractf(x); }
 };
@@ -77,6 +79,7 @@ struct Arith<double> {
   static __device__ __forceinline__ double clamp(double x, double lo, double hi) {
     return fmin(fmax(x, lo), hi);
   }
+  static __device__ __forceinline__ double clamp01(double x) { return fmin(fmax(x, 0.0), 1.0); }
   static __device__ __forceinline__ double fract(double x) { return __builtin_amdgcn_fract(x); }
 };
 

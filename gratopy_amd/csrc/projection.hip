@@ -502,6 +502,95 @@ __global__ __launch_bounds__(256, WAVES) void back_stack_kernel(Job<real> J, rea
   back_stack_tile<real, FAN, G, RP, CAP>(J, bx, blockIdx.y, blockIdx.z, a0, a1, part, band, sh);
 }
 
+// ---- slice-batched forward (fwd_stack_block) ---------------------------------
+// A gather: a lane owns one ray and reads the T columns of its strip in each
+// row, instead of scattering pixels into LDS slots as the bin groups above do.
+// The strip's weights are computed once for up to 8 slices, and the image comes
+// from LDS in 16-byte entries of slices.  What bounds it: per strip row T (4 G)
+// FMAs and LDS reads of 16 T G bytes a lane beside ~5 T instructions of weights
+// (fan: one v_rcp_f32 per column).  The parallel beam, whose rays are more than
+// a column apart, has two lanes on a bank in most reads and is held by them.
+// 32 x 2048^2, 1440 angles: fan 68.2 -> 28.6 ms, parallel beam 68.0 -> 31.1 ms;
+// 16 x 512^2 fan, 360 angles: float32 937 -> 476 us, float64 2030 -> 1150 us.
+//
+// Prologue: both image copies in entries of slices (block: 32 x 32 pixels of one
+// group), and, in the first layer of blocks, the angles sorted by their
+// direction (each thread counts the angles that come before its own).
+template <typename real>
+__global__ __launch_bounds__(256) void stack_images_kernel(Entry<real> *__restrict__ X,
+                                                           Entry<real> *__restrict__ Y,
+                                                           const real *__restrict__ img, Strides3 ii, int Nx,
+                                                           int Ny, int Nz, int *__restrict__ perm,
+                                                           const real *__restrict__ ofs, int Na) {
+  __shared__ Entry<real> tile[32][33];
+  const int q = (int)blockIdx.z - 1;
+  if (q < 0) {
+    // directions of the detector axis in [-2, 2): monotone in its angle
+    auto key = [&](int a) {
+      const float x = (float)ofs[8 * (int64_t)a], y = (float)ofs[8 * (int64_t)a + 1];
+      const float r = x / (fabsf(x) + fabsf(y));
+      return y < 0 ? r - 1 : 1 - r;
+    };
+    float *keys = reinterpret_cast<float *>(tile);
+    const int nb = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
+    for (int a0 = b * 256; a0 < Na; a0 += nb * 256) {
+      const int a = a0 + threadIdx.x;
+      const float own = a < Na ? key(a) : 0;
+      int rank = 0;
+      for (int c0 = 0; c0 < Na; c0 += 256) {
+        __syncthreads();
+        if (c0 + (int)threadIdx.x < Na) keys[threadIdx.x] = key(c0 + threadIdx.x);
+        __syncthreads();
+        const int n = min(256, Na - c0);
+#pragma unroll 8
+        for (int i = 0; i < n; ++i) {
+          const float k = keys[i];
+          rank += k < own || (!(own < k) && c0 + i < a);
+        }
+      }
+      if (a < Na) perm[rank] = a;
+    }
+    return;
+  }
+  const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
+  const int lx = threadIdx.x & 31, ly = threadIdx.x >> 5;
+  const bool x_first = ii.s0 <= ii.s1;
+  for (int k = ly; k < 32; k += 8) {
+    const int x = x0 + (x_first ? lx : k), y = y0 + (x_first ? k : lx);
+    if (x >= Nx || y >= Ny) continue;
+    Entry<real> e;
+#pragma unroll
+    for (int i = 0; i < kSlices<real>; ++i) {
+      const int z = q * kSlices<real> + i;
+      e.v[i] = z < Nz ? img[x * ii.s0 + y * ii.s1 + z * ii.s2] : (real)0;
+    }
+    tile[y - y0][x - x0] = e;
+  }
+  __syncthreads();
+  const Entry<real> zero{};
+  for (int k = ly; k < 32; k += 8) {
+    const int x = x0 + lx, y = y0 + k;
+    Entry<real> *row = X + ((int64_t)q * Ny + y) * (Nx + 1);
+    if (y < Ny && x < Nx) row[x] = tile[k][lx];
+    if (y < Ny && x == Nx - 1) row[Nx] = zero;
+  }
+  for (int k = ly; k < 32; k += 8) {
+    const int y = y0 + lx, x = x0 + k;
+    Entry<real> *row = Y + ((int64_t)q * Nx + x) * (Ny + 1);
+    if (x < Nx && y < Ny) row[y] = tile[lx][k];
+    if (x < Nx && y == Ny - 1) row[Ny] = zero;
+  }
+}
+
+template <typename real, bool FAN, int G, int H, int CAP, int WAVES>
+__global__ __launch_bounds__(256 * H, WAVES) void fwd_stack_kernel(Job<real> J, const int *perm, real *part,
+                                                               int nbands, int nrb) {
+  __shared__ FwdShared<real, G, CAP> sh;
+  const int band = blockIdx.x / nrb;
+  fwd_stack_block<real, FAN, G, H, CAP>(J, perm, blockIdx.x - band * nrb, blockIdx.y, blockIdx.z, band, nbands,
+                                     part, sh);
+}
+
 // ---------------------------------------------------------------------------
 // Single-line (impulse response) kernels for the sparse system matrix.
 // ---------------------------------------------------------------------------
@@ -772,6 +861,62 @@ static size_t back_need(int dtype, const Layout &L) {
   return s.g ? back_stack_ws(dtype, L, s) : back_ws(dtype, L);
 }
 
+// Slice-batched forward: g slice groups per lane, halves x 64 rays per block,
+// row bands.  g = 0: the launch shapes above.
+struct FwdStackShape {
+  int g, halves, bands;
+};
+
+static FwdStackShape fwd_stack_shape(int dtype, const Layout &L) {
+  FwdStackShape s{0, 1, 1};
+  const int slices = 16 / (int)elem_size(dtype);
+  if (!tuning().automatic || L.Nz == 1 || work_of(L) < 3e7) return s;
+  // From three slices on (two float64 slices of a parallel beam fill an entry).
+  // Start -> here, us: 512^2, 360 angles, 725 detectors: fan 2 / 3 / 4 / 8 slices
+  // 154 -> 201 / 209 -> 203 / 272 -> 206 / 458 -> 318, parallel beam 143 -> 150 /
+  // 190 -> 151 / 247 -> 154 / 423 -> 250.
+  if (L.Nz == 2 && (dtype == GT_FLOAT32 || L.fan)) return s;
+  // Fan strips are narrow on small detectors (two rays a column and fewer), and
+  // 64 rays span much of the fan: 256^2 x 8 with 363 detectors 103 -> 105 us.
+  if (L.fan && L.Ns <= 512) return s;
+  // The eight angles of a block share their windows: neighbours at 1/10 of an
+  // angle a pixel still fit (512^2 x 8, 50 angles: 119 -> 88 us, fan 130 -> 107).
+  if ((int64_t)L.Na * 12 < std::max(L.Nx, L.Ny)) return s;
+  if ((int64_t)(L.Nx + 1) * (L.Ny + 1) >= (int64_t)1 << 27) return s;  // a group's copy stays below 2^31 bytes
+  // 128 rays a block share their windows' ends; small detectors fill 64 better
+  // (7 x 301 x 257, 403 detectors: 83 us against 91).
+  s.halves = L.Ns <= 512 ? 1 : 2;
+  // Two groups per lane halve a ray's weights per slice; the parallel beam's are
+  // three additions in float32 and its LDS reads decide either way (2048^2 x 8:
+  // 8.1 ms with one, 8.4 with two; fan 9.7 against 8.5).
+  const int fill1 = (L.Nz + slices - 1) / slices, fill2 = (fill1 + 1) / 2 * 2;
+  s.g = (L.fan || dtype == GT_FLOAT64) && s.halves == 2 && fill2 * 100 <= fill1 * 115 ? 2 : 1;
+  // Row bands until the launch has about 3 blocks for each that fits the GPU
+  // (512^2 x 16 fan, 540 blocks: 701 / 604 / 484 / 476 us over 1 / 2 / 4 / 8;
+  // 512^2 x 4 parallel beam, 270 blocks: 344 / 207 / 154 / 155).
+  const int64_t blocks = (int64_t)((L.Ns + 64 * s.halves - 1) / (64 * s.halves)) *
+                         ((L.Na + kFwdAngles - 1) / kFwdAngles) * ((fill1 + s.g - 1) / s.g);
+  while (s.bands < 8 && blocks * s.bands < 2200) s.bands *= 2;
+  return s;
+}
+
+static size_t fwd_stack_copy(int dtype, int n0, int n1, int Nz, const FwdStackShape &s) {
+  const size_t slices = 16 / elem_size(dtype);
+  const size_t groups = ((size_t)Nz + slices * s.g - 1) / (slices * s.g) * s.g;
+  return align_up((size_t)16 * groups * n1 * (size_t)(n0 + 1));
+}
+
+static size_t fwd_stack_ws(int dtype, const Layout &L, const FwdStackShape &s) {
+  return align_up(sizeof(int) * (size_t)L.Na) + fwd_stack_copy(dtype, L.Nx, L.Ny, L.Nz, s) +
+         fwd_stack_copy(dtype, L.Ny, L.Nx, L.Nz, s) +
+         (s.bands > 1 ? align_up(elem_size(dtype) * (size_t)s.bands * L.Ns * L.Na * L.Nz) : 0);
+}
+
+static size_t fwd_need(int dtype, const Layout &L, int img_order) {
+  const FwdStackShape s = fwd_stack_shape(dtype, L);
+  return s.g ? fwd_stack_ws(dtype, L, s) : fwd_ws(dtype, L, img_order);
+}
+
 template <typename real>
 static Job<real> make_job(bool fan, const Layout &L, const real *ofs, const real *sdpd,
                           const real *geo) {
@@ -835,11 +980,62 @@ static int launch_fwd_group(hipStream_t st, const Job<real> &J, int nb, bool chu
   return GT_OK;
 }
 
+template <typename real, bool FAN, int G, int H, int CAP, int WAVES>
+static void launch_fwd_stack(hipStream_t st, const Job<real> &J, const int *perm, const FwdStackShape &sh,
+                             real *part) {
+  constexpr int slices = kSlices<real> * G;
+  const int nrb = (J.Ns + 64 * H - 1) / (64 * H);
+  const dim3 grid((unsigned)(nrb * sh.bands), (J.Na + kFwdAngles - 1) / kFwdAngles,
+                  (J.Nz + slices - 1) / slices);
+  hipLaunchKernelGGL((fwd_stack_kernel<real, FAN, G, H, CAP, WAVES>), grid, dim3(256 * H), 0, st, J, perm, part,
+                     sh.bands, nrb);
+}
+
+template <typename real, bool FAN>
+static int fwd_stack_impl(hipStream_t st, real *sino, const real *img, const real *ofs, const real *sdpd,
+                          const real *geo, const Layout &L, int sino_order, int img_order, char *w,
+                          const FwdStackShape &sh) {
+  constexpr int dtype = sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32;
+  const int groups = (L.Nz + kSlices<real> * sh.g - 1) / (kSlices<real> * sh.g) * sh.g;
+  int *perm = reinterpret_cast<int *>(w);
+  w += align_up(sizeof(int) * (size_t)L.Na);
+  Entry<real> *X = reinterpret_cast<Entry<real> *>(w);
+  w += fwd_stack_copy(dtype, L.Nx, L.Ny, L.Nz, sh);
+  Entry<real> *Y = reinterpret_cast<Entry<real> *>(w);
+  w += fwd_stack_copy(dtype, L.Ny, L.Nx, L.Nz, sh);
+  real *part = sh.bands > 1 ? reinterpret_cast<real *>(w) : nullptr;
+  hipLaunchKernelGGL(stack_images_kernel<real>, dim3((L.Nx + 31) / 32, (L.Ny + 31) / 32, groups + 1),
+                     dim3(256), 0, st, X, Y, img, order_strides(img_order, L.Nx, L.Ny, L.Nz), L.Nx, L.Ny,
+                     L.Nz, perm, ofs, L.Na);
+  Job<real> J = make_job<real>(FAN, L, ofs, sdpd, geo);
+  J.sino = sino;
+  J.so = order_strides(sino_order, L.Ns, L.Na, L.Nz);
+  J.imgX = X->v;
+  J.imgY = Y->v;
+  if (sh.g == 2 && sh.halves == 2)
+    launch_fwd_stack<real, FAN, 2, 2, 736, 6>(st, J, perm, sh, part);
+  else if (sh.g == 2)
+    launch_fwd_stack<real, FAN, 2, 1, 336, 6>(st, J, perm, sh, part);
+  else if (sh.halves == 2)
+    launch_fwd_stack<real, FAN, 1, 2, 1472, 6>(st, J, perm, sh, part);
+  else
+    launch_fwd_stack<real, FAN, 1, 1, 672, 6>(st, J, perm, sh, part);
+  if (part)
+    hipLaunchKernelGGL(band_reduce_kernel<real>, dim3((L.Ns + 255) / 256, L.Na, L.Nz), dim3(256), 0, st, J,
+                       part, sh.bands, nullptr, 1);
+  return check_launch(FAN ? "fan forward projection" : "radon forward projection");
+}
+
 template <typename real, bool FAN>
 static int fwd_impl(hipStream_t st, real *sino, const real *img, const real *ofs,
                     const real *sdpd, const real *geo, const Layout &L, int sino_order,
                     int img_order, void *ws, size_t ws_bytes) {
-  const size_t need = fwd_ws(sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32, L, img_order);
+  const int dtype = sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32;
+  const FwdStackShape ss = fwd_stack_shape(dtype, L);
+  if (ss.g && ws != nullptr && ws_bytes >= fwd_stack_ws(dtype, L, ss))
+    return fwd_stack_impl<real, FAN>(st, sino, img, ofs, sdpd, geo, L, sino_order, img_order,
+                                     static_cast<char *>(ws), ss);
+  const size_t need = fwd_ws(dtype, L, img_order);
   if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
   GT_REQUIRE(need == 0 || ws != nullptr, "workspace pointer is NULL");
   const Strides3 is = order_strides(img_order, L.Nx, L.Ny, L.Nz);
@@ -1031,7 +1227,7 @@ extern "C" size_t gt_projection_workspace_bytes(int geometry, int adjoint, int d
                                                 int Ny, int Ns, int Na, int Nz, int in_order) {
   if (Nx <= 0 || Ny <= 0 || Ns <= 0 || Na <= 0 || Nz <= 0) return 0;
   const Layout L{Nx, Ny, Ns, Na, Nz, geometry == GT_GEOMETRY_FAN};
-  return adjoint ? back_need(dtype, L) : fwd_ws(dtype, L, in_order);
+  return adjoint ? back_need(dtype, L) : fwd_need(dtype, L, in_order);
 }
 
 extern "C" int gt_projection_shape(int geometry, int adjoint, int Nx, int Ny, int Ns, int Na,

@@ -297,4 +297,545 @@ __device__ __forceinline__ void back_stack_tile(const Job<real> &J, int bx, int 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Forward projection.
+// ---------------------------------------------------------------------------
+// Image copies of the slice groups: x-fastest entries X[(q Ny + y)(Nx + 1) + x]
+// and y-fastest entries Y[(q Nx + x)(Ny + 1) + y]; the last entry of a row is
+// zero (reads outside the row take it).
+
+// One ray of a strip in the frame whose rows run along it: the strip's left
+// edge crosses row y at column u0 + m y, its right edge at v0 + n y.  Parallel
+// beam: a pixel d columns right of the left edge weighs 1 - |A d - 1|.  Fanbeam:
+// (1 - |A d / t - 1|) / t with t = t0 + t1 y + t2 d, the pixel's depth over the
+// source-detector distance; A, t0, t1 and t2 carry a common power of two that
+// makes t at least 1 over the image.
+struct StripRay {
+  double u0, m, v0, n, A, t0, t1, t2;
+};
+
+// One angle of the block: its table entries in double and the power of two
+// (0: none, a corner of the image is not in front of the source).
+struct FwdAngle {
+  double o[6], scale;
+  int a;
+};
+
+// The frame of a ray: rows along y (x fastest), or flipped.
+template <typename real>
+__device__ __forceinline__ bool strip_flipped(const Job<real> &J, const FwdAngle &r, double s) {
+  if (!J.fan) return fabs(r.o[0]) < fabs(r.o[1]);
+  const double d = s - (double)J.geo[5];
+  return !(fabs(r.o[4] + r.o[0] * d - r.o[2]) < fabs(r.o[5] + r.o[1] * d - r.o[3]));
+}
+
+template <typename real>
+__device__ __forceinline__ FwdAngle fwd_angle(const Job<real> &J, int a) {
+  FwdAngle r;
+  r.a = a;
+  r.scale = 1;
+  for (int i = 0; i < 6; ++i) r.o[i] = J.ofs[8 * (int64_t)a + i];
+  if (J.fan) {
+    // depth over source-detector distance, linear: least at a corner
+    const double R = J.geo[0], ddx = (r.o[4] - r.o[2]) / (R * R), ddy = (r.o[5] - r.o[3]) / (R * R);
+    const double t = (double)J.geo[1] / R - ddx * (double)J.geo[3] - ddy * (double)J.geo[4] +
+                     fmin(0.0, ddx * (J.Nx - 1)) + fmin(0.0, ddy * (J.Ny - 1));
+    r.scale = t > 1e-30 ? ldexp(1.0, max(0, 1 - ilogb(t))) : 0.0;
+  }
+  return r;
+}
+
+template <typename real, bool FAN>
+__device__ __forceinline__ StripRay strip_ray(const Job<real> &J, const FwdAngle &g, double s, bool flip) {
+  const double *o = g.o;
+  StripRay r;
+  if constexpr (!FAN) {
+    const double X = flip ? o[1] : o[0], Y = flip ? o[0] : o[1], i = 1.0 / X;
+    r.m = r.n = -Y * i;
+    const double c = (s - o[2]) * i, h = fabs(i);
+    r.u0 = c - h;
+    r.v0 = c + h;
+    r.A = fabs(X);
+    r.t0 = r.t1 = r.t2 = 0;
+  } else {
+    const double R = J.geo[0], dxi = J.geo[2], mid = J.geo[5];
+    const double midx = flip ? J.geo[4] : J.geo[3], midy = flip ? J.geo[3] : J.geo[4];
+    const double xd = flip ? o[1] : o[0], yd = flip ? o[0] : o[1];
+    const double qx = flip ? o[3] : o[2], qy = flip ? o[2] : o[3];
+    const double d0x = flip ? o[5] : o[4], d0y = flip ? o[4] : o[5];
+    double sl = s - 1, sr = s + 1;
+    double pl = (d0x + xd * (sl - mid) - qx) / (d0y + yd * (sl - mid) - qy);
+    double pr = (d0x + xd * (sr - mid) - qx) / (d0y + yd * (sr - mid) - qy);
+    if (qy * (pr - pl) > 0) {  // the rays run away from the source: rows lie at -qy of it
+      const double w = pl;
+      pl = pr;
+      pr = w;
+      sl = s + 1;
+    }
+    const double ddx = (d0x - qx) / (R * R), ddy = (d0y - qy) / (R * R);
+    r.m = pl;
+    r.n = pr;
+    r.u0 = qx + midx - pl * (midy + qy);
+    r.v0 = qx + midx - pr * (midy + qy);
+    r.A = g.scale * fabs(xd / (dxi * dxi) + (mid - sl) * ddx);
+    r.t0 = g.scale * (ddx * (r.u0 - midx) - ddy * midy + (double)J.geo[1] / R);
+    r.t1 = g.scale * (ddx * pl + ddy);
+    r.t2 = g.scale * ddx;
+  }
+  return r;
+}
+
+// Column of a strip's left edge along the rows: whole part and fraction.
+// Single precision carries 32.32 fixed point, two integer additions a row.
+template <typename real>
+struct StripColumn;
+
+template <>
+struct StripColumn<float> {
+  int64_t u, m;
+  __device__ __forceinline__ void start(double u0, double slope, int y) {
+    const double v = fma(slope, (double)y, u0), f = floor(v);
+    u = ((int64_t)(int)f << 32) + (int64_t)(uint32_t)((v - f) * 4294967296.0);
+    m = (int64_t)rint(slope * 4294967296.0);
+  }
+  __device__ __forceinline__ int whole() const { return (int)(u >> 32); }
+  // 1 - fraction: distance of the first whole column right of the edge
+  __device__ __forceinline__ float first() const { return fma((float)(uint32_t)u, -0x1p-32f, 1.0f); }
+  __device__ __forceinline__ void step() { u += m; }
+};
+
+template <>
+struct StripColumn<double> {
+  double u0, m, y;
+  __device__ __forceinline__ void start(double u, double slope, int y0) {
+    u0 = u;
+    m = slope;
+    y = y0;
+  }
+  __device__ __forceinline__ int whole() const { return (int)floor(fma(m, y, u0)); }
+  __device__ __forceinline__ double first() const { return 1.0 - Arith<double>::fract(fma(m, y, u0)); }
+  __device__ __forceinline__ void step() { y += 1; }
+};
+
+constexpr int kFwdAngles = 8;   // angles per block, neighbours in direction
+constexpr int kFwdKnot = 16;    // rows per interval of the window table
+constexpr int kFwdKnots = 256;  // intervals per table
+
+template <typename real, int G, int CAP>
+struct FwdShared {
+  Entry<real> buf[2][G * CAP];
+  int4 table[kFwdKnots];  // FwdChunk of each interval: first column, pitch, rows per chunk, taps
+  FwdAngle angle[kFwdAngles];
+  StripRay edge[2 * kFwdAngles];
+  int flips, irregular, first, last;
+};
+
+// Lane's ray within its wave's 64: a 16-byte LDS read is served in four
+// phases of 16 lanes, {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31} and the same of
+// the upper half (found by pairing lanes on one bank).  Each phase gets 16
+// neighbouring rays, whose entries then lie in different banks while rays are
+// at most a column apart.
+__device__ __forceinline__ int phase_ray(int lane) {
+  const int l = lane & 31;
+  int r;
+  if (l < 4)
+    r = l;
+  else if (l < 12)
+    r = l + 12;
+  else if (l < 16)
+    r = l - 8;
+  else if (l < 20)
+    r = l + 8;
+  else if (l < 28)
+    r = l - 12;
+  else
+    r = l;
+  return (lane & 32) + r;
+}
+
+// Rows [y, y + rows) of one window: image columns from (xw(y) >> 32) + lo on,
+// pitch of them, at most `taps` per ray.
+struct FwdChunk {
+  int y, rows, lo, pitch, taps;
+};
+
+// What a lane keeps of its ray, at the next row.
+template <typename real>
+struct LaneRay {
+  StripColumn<real> col;
+  real A, t0, t1, t2;
+  __device__ __forceinline__ void start(const StripRay &r, int y) {
+    col.start(r.u0, r.m, y);
+    A = (real)r.A;
+    t0 = (real)r.t0;
+    t1 = (real)r.t1;
+    t2 = (real)r.t2;
+  }
+};
+
+// Adds the strip rows of one chunk, T columns each (T = 0: chunk.taps): acc +=
+// w(x, y) image(x, y).  xw, xm: the window's 32.32 start column and its slant.
+template <typename real, bool FAN, int G, int T>
+__device__ __forceinline__ void strip_rows(LaneRay<real> &R, const FwdChunk &c, int64_t xw, int64_t xm,
+                                           LdsEntry<real> buf, int plane, real (&acc)[G][kSlices<real>]) {
+  using A = Arith<real>;
+  int base = 1 - c.lo;
+  real y = (real)c.y;
+#pragma unroll 1
+  for (int r = 0; r < c.rows; ++r) {
+    const LdsEntry<real> p = buf + (R.col.whole() + (base - (int)(xw >> 32)));
+    const real d = R.col.first();
+    real n = R.A * d, t = FAN ? fma(d, R.t2, fma(y, R.t1, R.t0)) : (real)0;
+    auto weight = [&] {
+      real w;
+      if constexpr (FAN) {
+        const real q = A::rcp_positive(t), e = fma(n, q, (real)-1);
+        w = A::clamp01(fma(-fabs(e), q, q));
+        t += R.t2;
+      } else {
+        w = A::clamp01((real)1 - fabs(n - (real)1));
+      }
+      n += R.A;
+      return w;
+    };
+    auto add = [&](real w, int i) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const Entry<real> e = lds_entry<real>(p + g * plane + i);
+#pragma unroll
+        for (int z = 0; z < kSlices<real>; ++z) acc[g][z] = fma(w, e.v[z], acc[g][z]);
+      }
+    };
+    if constexpr (T > 0) {
+      real w[T];
+#pragma unroll
+      for (int i = 0; i < T; ++i) w[i] = weight();
+#pragma unroll
+      for (int i = 0; i < T; ++i) add(w[i], i);
+    } else {
+#pragma unroll 1
+      for (int i = 0; i < c.taps; ++i) add(weight(), i);
+    }
+    R.col.step();
+    base += c.pitch;
+    xw += xm;
+    y += 1;
+  }
+}
+
+// The same rows without windows (they do not fit LDS, or the ray leaves the
+// block's frame): every pixel of the strip, read from the image copy.
+template <typename real, bool FAN, int G>
+__device__ __forceinline__ void strip_direct(const StripRay &R, int y0, int y1, const Entry<real> *img,
+                                             int64_t quad, int Nxx, real (&acc)[G][kSlices<real>]) {
+#pragma unroll 1
+  for (int y = y0; y < y1; ++y) {
+    const double u = fma(R.m, (double)y, R.u0), v = fma(R.n, (double)y, R.v0);
+    // whole columns strictly inside (u, v) and the image; the comparisons keep
+    // infinities and NaN away from the conversions
+    if (!(u < (double)Nxx && v > -1.0)) continue;
+    const int xl = u > -1.0 ? (int)floor(u) + 1 : 0;
+    const int xh = v < (double)Nxx ? (int)ceil(v) - 1 : Nxx - 1;
+    const Entry<real> *row = img + (int64_t)y * (Nxx + 1);
+#pragma unroll 1
+    for (int x = xl; x <= xh; ++x) {
+      const double d = (double)x - u;
+      real w;
+      if constexpr (FAN) {
+        const real q = (real)1 / (real)(R.t0 + R.t1 * y + R.t2 * d);
+        w = ((real)1 - fabs(fma((real)(R.A * d), q, (real)-1))) * q;
+      } else {
+        w = (real)1 - fabs((real)(R.A * d - 1.0));
+      }
+      w = w > (real)0 ? w : (real)0;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const Entry<real> e = row[g * quad + x];
+#pragma unroll
+        for (int z = 0; z < kSlices<real>; ++z) acc[g][z] = fma(w, e.v[z], acc[g][z]);
+      }
+    }
+  }
+}
+
+// Results of one ray in G slice groups: band partials, or the projection with
+// its scale and epilogue.
+template <typename real, bool FAN, int G>
+__device__ __forceinline__ void strip_store(const Job<real> &J, int s, int a, int zb, int band, real *part,
+                                            real scale, const real (&sum)[G][kSlices<real>]) {
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int z = 0; z < kSlices<real>; ++z) {
+      const int zz = (zb * G + g) * kSlices<real> + z;
+      if (zz >= J.Nz) continue;
+      const real v = sum[g][z] * scale;
+      if (part)
+        part[(((int64_t)band * J.Nz + zz) * J.Na + a) * J.Ns + s] = v;
+      else if (FAN)
+        fan_store(J, s, a, zz, v);
+      else
+        store_fwd(J, s, a, zz, v * radon_scale(J));
+    }
+}
+
+// Forward projection of 64 H rays at kFwdAngles angles (neighbours in
+// direction: perm lists the angles sorted by it) in G slice groups.  The rays
+// walk the rows of their frame together: per chunk of rows the block copies
+// the columns that its rays can meet into LDS (slanted windows, the next chunk
+// loading while the current one is summed), and every lane adds the T columns
+// of each strip row, weights computed once for all slices.  Wave w: rays 64
+// (w % H) .. + 63, angles 2 (w / H) and the next.
+template <typename real, bool FAN, int G, int H, int CAP>
+__device__ __forceinline__ void fwd_stack_block(const Job<real> &J, const int *perm, int rb, int ag, int zb,
+                                                int band, int nbands, real *part,
+                                                FwdShared<real, G, CAP> &sh) {
+  using E = Entry<real>;
+  constexpr int ZV = kSlices<real>;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int first = rb * 64 * H, nray = min(64 * H, J.Ns - first);
+  const int s_own = first + (wv % H) * 64 + phase_ray(lane), s = min(s_own, J.Ns - 1);
+  const double s_mid = first + 0.5 * (nray - 1);
+  const int g0 = ag * kFwdAngles, na = min(kFwdAngles, J.Na - g0);
+  const int mine = 2 * (wv / H);  // the wave's first angle in the group
+  if (tid == 0) sh.flips = 0;
+  __syncthreads();
+  if (tid < na) {
+    const FwdAngle r = fwd_angle(J, perm[g0 + tid]);
+    sh.angle[tid] = r;
+    if (strip_flipped(J, r, s_mid)) atomicOr(&sh.flips, 1 << tid);
+  }
+  __syncthreads();
+  const int flips = __builtin_amdgcn_readfirstlane(sh.flips);
+
+  // runs of angles with one frame (nearly always the whole group)
+  for (int sub = 0, sub_end; sub < na; sub = sub_end) {
+    const bool flip = (flips >> sub) & 1;
+    sub_end = sub + 1;
+    while (sub_end < na && (bool)((flips >> sub_end) & 1) == flip) ++sub_end;
+    const int Nxx = flip ? J.Ny : J.Nx, Nyy = flip ? J.Nx : J.Ny;
+    const int y0 = (int)((int64_t)Nyy * band / nbands), y1 = (int)((int64_t)Nyy * (band + 1) / nbands);
+    const int64_t quad = (int64_t)Nyy * (Nxx + 1);
+    const E *img = reinterpret_cast<const E *>(flip ? J.imgY : J.imgX) + (int64_t)zb * G * quad;
+
+    __syncthreads();  // the previous run is done with the tables
+    if (tid == 0) {
+      sh.irregular = 0;
+      sh.first = kFwdKnots;
+      sh.last = -1;
+    }
+    __syncthreads();
+    const int nedge = 2 * (sub_end - sub);
+    if (tid < nedge) {
+      const FwdAngle &g = sh.angle[sub + (tid >> 1)];
+      const double se = (tid & 1) ? first + nray - 1 : first;
+      const StripRay r = strip_ray<real, FAN>(J, g, se, flip);
+      sh.edge[tid] = r;
+      bool ok = g.scale > 0 && fabs(r.m) < 4 && fabs(r.n) < 4 && fabs(r.u0) < 1e6 && fabs(r.v0) < 1e6;
+      if constexpr (FAN) {  // the edge rays reach the rows on the middle ray's side of the source
+        const double yd = flip ? g.o[0] : g.o[1], d0 = flip ? g.o[4] - g.o[2] : g.o[5] - g.o[3];
+        const double mid = J.geo[5], c = d0 + yd * (s_mid - mid);
+        ok = ok && (d0 + yd * (se - 1 - mid)) * c > 0 && (d0 + yd * (se + 1 - mid)) * c > 0;
+      }
+      if (!ok) atomicOr(&sh.irregular, 1);
+    }
+    __syncthreads();
+    // the windows' common slant: start column (xb + y xm) >> 32
+    const StripRay &e0 = sh.edge[0], &e1 = sh.edge[nedge - 1];
+    const int64_t xm = (int64_t)rint(0.5 * (e0.m + e1.m) * 4294967296.0);
+    const int64_t xb = (int64_t)rint(0.5 * (e0.u0 + e1.u0)) << 32;
+    // Window of rows [16 k, 16 k + 16): (first column, pitch, rows per chunk,
+    // taps), rows = 0 where no ray meets the image.  Every edge is linear along
+    // the rows, so the extremes lie at the interval's ends; it holds all taps of
+    // every ray, with one whole column to spare on each side for the rounding.
+    auto interval = [&](int k) {
+      double lo = 1e30, hi = -1e30, w = 0, xl = 1e30, xr = -1e30;
+      for (int end = 0; end < 2; ++end) {
+        const int y = (k + end) * kFwdKnot;
+        const double c = (double)(xb + y * xm) * (1.0 / 4294967296.0);
+        for (int i = 0; i < nedge; ++i) {
+          const StripRay &r = sh.edge[i];
+          const double u = fma(r.m, (double)y, r.u0), v = fma(r.n, (double)y, r.v0);
+          lo = fmin(lo, u - c);
+          hi = fmax(hi, u - c);
+          xl = fmin(xl, u);
+          xr = fmax(xr, v);
+          w = fmax(w, v - u);
+        }
+      }
+      const int l = (int)floor(lo) - 1, taps = (int)floor(w + 1e-3) + 1;
+      const int pitch = (int)floor(hi) + taps + 2 - l;
+      return make_int4(l, pitch, xr > -1 && xl < Nxx ? min(max(CAP / pitch, 1), kFwdKnot) : 0, taps);
+    };
+    const int k0 = y0 / kFwdKnot, k_end = (y1 + kFwdKnot - 1) / kFwdKnot;
+    // the first table, and the check of every interval's width
+    auto fill = [&](int kb) {
+      if (tid < min(kFwdKnots, k_end - kb)) {
+        const int4 t = interval(kb + tid);
+        sh.table[tid] = t;
+        if (t.z) {
+          atomicMin(&sh.first, tid);
+          atomicMax(&sh.last, tid);
+          if (t.y > CAP) atomicOr(&sh.irregular, 2);
+        }
+      }
+    };
+    if (!sh.irregular) {
+      for (int k = k0 + kFwdKnots + tid; k < k_end; k += 256 * H) {
+        const int4 t = interval(k);
+        if (t.z && t.y > CAP) atomicOr(&sh.irregular, 2);
+      }
+      fill(k0);
+    }
+    __syncthreads();
+    const int irregular = __builtin_amdgcn_readfirstlane(sh.irregular);
+    real tot[2][G][ZV];
+    bool active[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      active[e] = mine + e >= sub && mine + e < sub_end;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int z = 0; z < ZV; ++z) tot[e][g][z] = 0;
+    }
+    // buffers over the first and the last group's copy
+    const __amdgpu_buffer_rsrc_t rs0 =
+        __builtin_amdgcn_make_buffer_rsrc((void *)img, (short)0, (int)(quad * 16), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc((void *)(img + (G - 1) * quad),
+                                                                         (short)0, (int)(quad * 16), 0x00020000);
+    for (int kb = irregular ? k_end : k0; kb < k_end; kb += kFwdKnots) {
+      if (kb > k0) {
+        __syncthreads();
+        if (tid == 0) {
+          sh.first = kFwdKnots;
+          sh.last = -1;
+        }
+        __syncthreads();
+        fill(kb);
+        __syncthreads();
+      }
+      const int c_end = __builtin_amdgcn_readfirstlane(sh.last) + 1;
+      int ci = __builtin_amdgcn_readfirstlane(sh.first);
+      if (ci >= c_end) continue;
+      const int y_end = min((kb + c_end) * kFwdKnot, y1);
+      int cy = max((kb + ci) * kFwdKnot, y0);  // next chunk's first row, in interval ci
+      auto next = [&]() {
+        FwdChunk c{cy, 0, 0, 0, 0};
+        if (cy >= y_end) return c;
+        const int4 t = sh.table[ci];
+        const int ye = min((kb + ci + 1) * kFwdKnot, y1);
+        c.lo = __builtin_amdgcn_readfirstlane(t.x);
+        c.pitch = __builtin_amdgcn_readfirstlane(t.y);
+        c.rows = min(ye - cy, max(__builtin_amdgcn_readfirstlane(t.z), 1));
+        c.taps = __builtin_amdgcn_readfirstlane(t.w);
+        cy += c.rows;
+        ci += cy == ye;
+        return c;
+      };
+      auto stage = [&](const FwdChunk &c, E *dst) {
+        // row r of group g is copied by wave (r G + g) % 4H; columns outside the
+        // image take the row's zero entry
+        for (int it = wv; it < c.rows * G; it += 4 * H) {
+          const int r = it / G, g = it % G, y = c.y + r;
+          const int x0 = (int)((xb + y * xm) >> 32) + c.lo, row = y * (Nxx + 1);
+          E *to = dst + g * CAP + r * c.pitch;
+          for (int base = 0; base < c.pitch; base += 64) {
+            const int j = base + lane;
+            if (j < c.pitch) {
+              const int at = (row + (int)min((uint32_t)(x0 + j), (uint32_t)Nxx)) * 16;
+              auto *lds = (__attribute__((address_space(3))) void *)(to + base);
+              if (G == 1 || g == 0)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs0, lds, 16, at, 0, 0, 0);
+              else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs1, lds, 16, at, 0, 0, 0);
+            }
+          }
+        }
+      };
+      LaneRay<real> ray[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        if (active[e])
+          ray[e].start(strip_ray<real, FAN>(J, sh.angle[mine + e], s, flip), cy);
+      FwdChunk cur = next();
+      int which = 0;
+      stage(cur, sh.buf[0]);
+      while (cur.rows) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's copies have landed
+        __syncthreads();                     // everybody's have; the other buffer is free
+        const FwdChunk nxt = next();
+        if (nxt.rows) stage(nxt, sh.buf[which ^ 1]);
+        const LdsEntry<real> buf = (LdsEntry<real>)sh.buf[which];
+        const int64_t xw = xb + cur.y * xm;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          if (!active[e]) continue;
+          real acc[G][ZV];
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int z = 0; z < ZV; ++z) acc[g][z] = 0;
+          switch (cur.taps) {
+            case 1:
+              strip_rows<real, FAN, G, 1>(ray[e], cur, xw, xm, buf, CAP, acc);
+              break;
+            case 2:
+              strip_rows<real, FAN, G, 2>(ray[e], cur, xw, xm, buf, CAP, acc);
+              break;
+            case 3:
+              strip_rows<real, FAN, G, 3>(ray[e], cur, xw, xm, buf, CAP, acc);
+              break;
+            case 4:
+              strip_rows<real, FAN, G, 4>(ray[e], cur, xw, xm, buf, CAP, acc);
+              break;
+            default:
+              strip_rows<real, FAN, G, 0>(ray[e], cur, xw, xm, buf, CAP, acc);
+          }
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int z = 0; z < ZV; ++z) tot[e][g][z] += acc[g][z];
+        }
+        which ^= 1;
+        cur = nxt;
+      }
+    }
+    // Results, and the rays to take without windows: those of an irregular run
+    // and, whatever the pixel, those that met a value which is not finite (a tap
+    // of zero weight may lie outside the strip).
+    bool again[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      again[e] = false;
+      if (!active[e] || s_own >= J.Ns) continue;
+      real check = 0;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int z = 0; z < ZV; ++z) check = fma(tot[e][g][z], (real)0, check);
+      again[e] = irregular || check != (real)0;
+      if (!again[e])
+        strip_store<real, FAN, G>(J, s, sh.angle[mine + e].a, zb, band, part, (real)sh.angle[mine + e].scale,
+                                  tot[e]);
+    }
+#pragma unroll 1
+    for (int e = 0; e < 2; ++e) {
+      if (!(e ? again[1] : again[0])) continue;
+      FwdAngle g = sh.angle[mine + e];
+      g.scale = 1;
+      // rays that leave the block's frame take their own, in every row band alike
+      const bool f = irregular & 1 ? strip_flipped(J, g, s) : flip;
+      const int nx = f ? J.Ny : J.Nx, ny = f ? J.Nx : J.Ny;
+      const int64_t qd = (int64_t)ny * (nx + 1);
+      real sum[G][ZV] = {};
+      strip_direct<real, FAN, G>(strip_ray<real, FAN>(J, g, s, f), (int)((int64_t)ny * band / nbands),
+                                 (int)((int64_t)ny * (band + 1) / nbands),
+                                 reinterpret_cast<const E *>(f ? J.imgY : J.imgX) + (int64_t)zb * G * qd, qd, nx,
+                                 sum);
+      strip_store<real, FAN, G>(J, s, g.a, zb, band, part, (real)1, sum);
+    }
+  }
+}
+
 }  // namespace gt
