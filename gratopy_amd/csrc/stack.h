@@ -21,10 +21,22 @@ struct alignas(16) Entry {
 template <typename real>
 using LdsEntry = const __attribute__((address_space(3))) Entry<real> *;
 
+// What one LDS read of a strip walk returns: an entry of slices, or a single
+// slice's value.
+template <typename real, int Z>
+struct Slices {
+  real v[Z];
+};
+
 template <typename real>
-__device__ __forceinline__ Entry<real> lds_entry(LdsEntry<real> p) {
+__device__ __forceinline__ Slices<real, kSlices<real>> lds_slices(LdsEntry<real> p) {
   typedef real vec __attribute__((ext_vector_type(kSlices<real>)));
-  return __builtin_bit_cast(Entry<real>, *(const __attribute__((address_space(3))) vec *)p);
+  return __builtin_bit_cast(Slices<real, kSlices<real>>, *(const __attribute__((address_space(3))) vec *)p);
+}
+
+template <typename real>
+__device__ __forceinline__ Slices<real, 1> lds_slices(const __attribute__((address_space(3))) real *p) {
+  return {{*p}};
 }
 
 // ---------------------------------------------------------------------------
@@ -56,9 +68,8 @@ struct alignas(sizeof(real) * 8) TileWindow {
 };
 
 template <typename real, bool FAN, int TX, int TY>
-__device__ __forceinline__ TileWindow<real> tile_window(const Job<real> &J, int a, int xa, int ya,
-                                                        int cap) {
-  const AngleRec<real> c = J.tab[a];
+__device__ __forceinline__ TileWindow<real> tile_window(const Job<real> &J, const AngleRec<real> &c, int xa,
+                                                        int ya, int cap) {
   const double mid = FAN ? (double)J.geo[5] + 2.0 : 0.0;
   const double c0 = c.c[0], c1 = c.c[1], c2 = c.c[2];
   const double c3 = c.c[3], c4 = c.c[4], c5 = c.c[5];
@@ -99,13 +110,11 @@ __device__ __forceinline__ TileWindow<real> tile_window(const Job<real> &J, int 
 
 // Adds one angle to the lane's RP pixels of G slice groups.  STAGED:
 // win is the angle's window in LDS (planes of `plane` entries per group);
-// otherwise row + g quad are the padded sinogram rows in memory, read with the
-// coordinate clamped to [0.5, Ns + 2.5].
-template <typename real, bool FAN, int G, int RP, bool STAGED>
-__device__ __forceinline__ void stack_angle(const TileWindow<real> &W, real dx, real dy,
-                                            LdsEntry<real> win, int plane,
-                                            const Entry<real> *row, int64_t quad, real mid, real hi,
-                                            real (&acc)[RP][G][kSlices<real>]) {
+// otherwise bin(g, i) reads entry i of group g's padded sinogram row from
+// memory, with the coordinate clamped to [0.5, Ns + 2.5].
+template <typename real, bool FAN, int G, int RP, bool STAGED, typename Lds, typename Bin, int Z>
+__device__ __forceinline__ void stack_angle(const TileWindow<real> &W, real dx, real dy, Lds win, int plane,
+                                            Bin bin, real mid, real hi, real (&acc)[RP][G][Z]) {
   using A = Arith<real>;
   const real t0 = fma(W.c0, dx, fma(W.c1, dy, W.k0));
   const real q0 = FAN ? fma(W.k3, dx, fma(W.k4, dy, W.k1)) : t0;
@@ -134,21 +143,21 @@ __device__ __forceinline__ void stack_angle(const TileWindow<real> &W, real dx, 
   }
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    Entry<real> e0[RP], e1[RP];
+    Slices<real, Z> e0[RP], e1[RP];
 #pragma unroll
     for (int r = 0; r < RP; ++r) {
-      if (STAGED) {
-        e0[r] = lds_entry<real>(win + g * plane + ix[r]);
-        e1[r] = lds_entry<real>(win + g * plane + ix[r] + 1);
+      if constexpr (STAGED) {
+        e0[r] = lds_slices<real>(win + g * plane + ix[r]);
+        e1[r] = lds_slices<real>(win + g * plane + ix[r] + 1);
       } else {
-        e0[r] = row[g * quad + ix[r]];
-        e1[r] = row[g * quad + ix[r] + 1];
+        e0[r] = bin(g, ix[r]);
+        e1[r] = bin(g, ix[r] + 1);
       }
     }
 #pragma unroll
     for (int r = 0; r < RP; ++r)
 #pragma unroll
-      for (int z = 0; z < kSlices<real>; ++z)
+      for (int z = 0; z < Z; ++z)
         acc[r][g][z] = fma(w1[r], e1[r].v[z], fma(w0[r], e0[r].v[z], acc[r][g][z]));
   }
 }
@@ -201,7 +210,7 @@ __device__ __forceinline__ void back_stack_tile(const Job<real> &J, int bx, int 
     {
       int n = 0;
       if (tid < nb) {
-        const TileWindow<real> W = tile_window<real, FAN, T::kX, T::kY>(J, ab + tid, xa, ya, CAP);
+        const TileWindow<real> W = tile_window<real, FAN, T::kX, T::kY>(J, J.tab[ab + tid], xa, ya, CAP);
         sh.win[tid] = W;
         n = W.n;
       }
@@ -252,12 +261,12 @@ __device__ __forceinline__ void back_stack_tile(const Job<real> &J, int bx, int 
       if (!direct) {
 #pragma unroll 1
         for (int l = i0; l < end; ++l, cur += width)
-          stack_angle<real, FAN, G, RP, true>(sh.win[l], dx, dy, cur, CAP, nullptr, 0, mid, hi, acc);
+          stack_angle<real, FAN, G, RP, true>(sh.win[l], dx, dy, cur, CAP, nullptr, mid, hi, acc);
       } else {
 #pragma unroll 1
         for (int l = i0; l < end; ++l, cur += width)
           if (__builtin_amdgcn_readfirstlane(sh.win[l].n))
-            stack_angle<real, FAN, G, RP, true>(sh.win[l], dx, dy, cur, CAP, nullptr, 0, mid, hi, acc);
+            stack_angle<real, FAN, G, RP, true>(sh.win[l], dx, dy, cur, CAP, nullptr, mid, hi, acc);
       }
       which ^= 1;
     }
@@ -265,9 +274,12 @@ __device__ __forceinline__ void back_stack_tile(const Job<real> &J, int bx, int 
 #pragma unroll 1
       for (int l = 0; l < nb; ++l)
         if (__builtin_amdgcn_readfirstlane(sh.win[l].n) == 0)
-          stack_angle<real, FAN, G, RP, false>(sh.win[l], dx, dy, nullptr, 0,
-                                                   S + (int64_t)(ab + l) * Nsp, quad, mid,
-                                                   hi, acc);
+          stack_angle<real, FAN, G, RP, false>(
+              sh.win[l], dx, dy, LdsEntry<real>(), 0,
+              [&](int g, int i) {
+                return __builtin_bit_cast(Slices<real, ZV>, S[(int64_t)(ab + l) * Nsp + g * quad + i]);
+              },
+              mid, hi, acc);
     }
 #pragma unroll
     for (int r = 0; r < RP; ++r)
@@ -321,12 +333,26 @@ struct FwdAngle {
   int a;
 };
 
-// The frame of a ray: rows along y (x fastest), or flipped.
+// The frame of a ray: rows along y (x fastest), or flipped, where an edge of its
+// strip is flatter than that (gratopy/fanbeam.cl:150-165).
 template <typename real>
 __device__ __forceinline__ bool strip_flipped(const Job<real> &J, const FwdAngle &r, double s) {
   if (!J.fan) return fabs(r.o[0]) < fabs(r.o[1]);
+  auto steep = [&](double d) {
+    return fabs(r.o[4] + r.o[0] * d - r.o[2]) < fabs(r.o[5] + r.o[1] * d - r.o[3]);
+  };
   const double d = s - (double)J.geo[5];
-  return !(fabs(r.o[4] + r.o[0] * d - r.o[2]) < fabs(r.o[5] + r.o[1] * d - r.o[3]));
+  return !(steep(d - 1) && steep(d + 1));
+}
+
+// Whether both edges of a fan ray's strip run from the source to the rows at its
+// image side, the side for which strip_ray tells left from right (in its own
+// frame a ray of a wide fan may leave on either side of the source's row).
+template <typename real>
+__device__ __forceinline__ bool strip_forward(const Job<real> &J, const FwdAngle &r, double s, bool flip) {
+  const double yd = flip ? r.o[0] : r.o[1], qy = flip ? r.o[2] : r.o[3], d0 = (flip ? r.o[4] : r.o[5]) - qy;
+  const double d = s - (double)J.geo[5];
+  return qy * (d0 + yd * (d - 1)) < 0 && qy * (d0 + yd * (d + 1)) < 0;
 }
 
 template <typename real>
@@ -475,15 +501,15 @@ struct LaneRay {
 
 // Adds the strip rows of one chunk, T columns each (T = 0: chunk.taps): acc +=
 // w(x, y) image(x, y).  xw, xm: the window's 32.32 start column and its slant.
-template <typename real, bool FAN, int G, int T>
+template <typename real, bool FAN, int G, int T, typename Lds, int Z>
 __device__ __forceinline__ void strip_rows(LaneRay<real> &R, const FwdChunk &c, int64_t xw, int64_t xm,
-                                           LdsEntry<real> buf, int plane, real (&acc)[G][kSlices<real>]) {
+                                           Lds buf, int plane, real (&acc)[G][Z]) {
   using A = Arith<real>;
   int base = 1 - c.lo;
   real y = (real)c.y;
 #pragma unroll 1
   for (int r = 0; r < c.rows; ++r) {
-    const LdsEntry<real> p = buf + (R.col.whole() + (base - (int)(xw >> 32)));
+    const Lds p = buf + (R.col.whole() + (base - (int)(xw >> 32)));
     const real d = R.col.first();
     real n = R.A * d, t = FAN ? fma(d, R.t2, fma(y, R.t1, R.t0)) : (real)0;
     auto weight = [&] {
@@ -501,9 +527,9 @@ __device__ __forceinline__ void strip_rows(LaneRay<real> &R, const FwdChunk &c, 
     auto add = [&](real w, int i) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const Entry<real> e = lds_entry<real>(p + g * plane + i);
+        const Slices<real, Z> e = lds_slices<real>(p + g * plane + i);
 #pragma unroll
-        for (int z = 0; z < kSlices<real>; ++z) acc[g][z] = fma(w, e.v[z], acc[g][z]);
+        for (int z = 0; z < Z; ++z) acc[g][z] = fma(w, e.v[z], acc[g][z]);
       }
     };
     if constexpr (T > 0) {
@@ -524,10 +550,11 @@ __device__ __forceinline__ void strip_rows(LaneRay<real> &R, const FwdChunk &c, 
 }
 
 // The same rows without windows (they do not fit LDS, or the ray leaves the
-// block's frame): every pixel of the strip, read from the image copy.
-template <typename real, bool FAN, int G>
-__device__ __forceinline__ void strip_direct(const StripRay &R, int y0, int y1, const Entry<real> *img,
-                                             int64_t quad, int Nxx, real (&acc)[G][kSlices<real>]) {
+// block's frame): every pixel of the strip, as pixel(g, y, x) reads group g's
+// from memory.
+template <typename real, bool FAN, int G, typename Pixel, int Z>
+__device__ __forceinline__ void strip_direct(const StripRay &R, int y0, int y1, int Nxx, Pixel pixel,
+                                             real (&acc)[G][Z]) {
 #pragma unroll 1
   for (int y = y0; y < y1; ++y) {
     const double u = fma(R.m, (double)y, R.u0), v = fma(R.n, (double)y, R.v0);
@@ -536,7 +563,6 @@ __device__ __forceinline__ void strip_direct(const StripRay &R, int y0, int y1, 
     if (!(u < (double)Nxx && v > -1.0)) continue;
     const int xl = u > -1.0 ? (int)floor(u) + 1 : 0;
     const int xh = v < (double)Nxx ? (int)ceil(v) - 1 : Nxx - 1;
-    const Entry<real> *row = img + (int64_t)y * (Nxx + 1);
 #pragma unroll 1
     for (int x = xl; x <= xh; ++x) {
       const double d = (double)x - u;
@@ -550,9 +576,9 @@ __device__ __forceinline__ void strip_direct(const StripRay &R, int y0, int y1, 
       w = w > (real)0 ? w : (real)0;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const Entry<real> e = row[g * quad + x];
+        const auto e = pixel(g, y, x);
 #pragma unroll
-        for (int z = 0; z < kSlices<real>; ++z) acc[g][z] = fma(w, e.v[z], acc[g][z]);
+        for (int z = 0; z < Z; ++z) acc[g][z] = fma(w, e.v[z], acc[g][z]);
       }
     }
   }
@@ -632,11 +658,7 @@ __device__ __forceinline__ void fwd_stack_block(const Job<real> &J, const int *p
       const StripRay r = strip_ray<real, FAN>(J, g, se, flip);
       sh.edge[tid] = r;
       bool ok = g.scale > 0 && fabs(r.m) < 4 && fabs(r.n) < 4 && fabs(r.u0) < 1e6 && fabs(r.v0) < 1e6;
-      if constexpr (FAN) {  // the edge rays reach the rows on the middle ray's side of the source
-        const double yd = flip ? g.o[0] : g.o[1], d0 = flip ? g.o[4] - g.o[2] : g.o[5] - g.o[3];
-        const double mid = J.geo[5], c = d0 + yd * (s_mid - mid);
-        ok = ok && (d0 + yd * (se - 1 - mid)) * c > 0 && (d0 + yd * (se + 1 - mid)) * c > 0;
-      }
+      ok = ok && (!FAN || strip_forward(J, g, se, flip));
       if (!ok) atomicOr(&sh.irregular, 1);
     }
     __syncthreads();
@@ -828,11 +850,11 @@ __device__ __forceinline__ void fwd_stack_block(const Job<real> &J, const int *p
       const bool f = irregular & 1 ? strip_flipped(J, g, s) : flip;
       const int nx = f ? J.Ny : J.Nx, ny = f ? J.Nx : J.Ny;
       const int64_t qd = (int64_t)ny * (nx + 1);
+      const E *from = reinterpret_cast<const E *>(f ? J.imgY : J.imgX) + (int64_t)zb * G * qd;
       real sum[G][ZV] = {};
-      strip_direct<real, FAN, G>(strip_ray<real, FAN>(J, g, s, f), (int)((int64_t)ny * band / nbands),
-                                 (int)((int64_t)ny * (band + 1) / nbands),
-                                 reinterpret_cast<const E *>(f ? J.imgY : J.imgX) + (int64_t)zb * G * qd, qd, nx,
-                                 sum);
+      strip_direct<real, FAN>(strip_ray<real, FAN>(J, g, s, f), (int)((int64_t)ny * band / nbands),
+                              (int)((int64_t)ny * (band + 1) / nbands), nx,
+                              [&](int gr, int y, int x) { return from[gr * qd + (int64_t)y * (nx + 1) + x]; }, sum);
       strip_store<real, FAN, G>(J, s, g.a, zb, band, part, (real)1, sum);
     }
   }

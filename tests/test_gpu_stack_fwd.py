@@ -35,6 +35,7 @@ STACKS = [
     ("radon", (128, 128), 8, 240, 23, F32, "F", {}),       # strips many columns wide
     ("radon", (1600, 90), 3, 140, 64, F32, "F", {}),       # windows wider than LDS
     ("fan", (300, 40), 8, 320, 540, F32, "F", dict(detector_width=9000.0)),  # a fan of 150 degrees
+    ("fan", (40, 40), 8, 2400, 520, F64, "F", dict(detector_width=1200.0)),
     ("fan", (128, 128), 8, 260, 600, F32, "C", dict(midpoint_shift=(9.0, -14.0), detector_shift=11.0,
                                                     reverse_detector=True)),
     ("radon", (128, 128), 8, 260, 200, F64, "C", dict(midpoint_shift=(9.0, -14.0), detector_shift=11.0)),
