@@ -71,6 +71,11 @@ class Queue:
             return self.stream
         return torch.cuda.current_stream(self.device)
 
+    def current_handle(self) -> int:
+        """Handle of torch's current stream on this device, without the Stream
+        object around it."""
+        return torch._C._cuda_getCurrentRawStream(self.device.index)
+
     def handle(self) -> int:
         return self.torch_stream().cuda_stream
 
@@ -93,7 +98,7 @@ def is_c_contiguous(t) -> bool:
 
 
 def is_f_contiguous(t) -> bool:
-    return t.permute(*reversed(range(t.dim()))).is_contiguous()
+    return (t.t() if t.dim() == 2 else t.permute(*reversed(range(t.dim())))).is_contiguous()
 
 
 def order_of(t) -> str:
@@ -119,7 +124,11 @@ def empty(shape, dtype, order="F", device=None):
     tdt = to_torch_dtype(dtype)
     if order.upper() == "C":
         return torch.empty(shape, dtype=tdt, device=device)
-    return torch.empty(shape[::-1], dtype=tdt, device=device).permute(*reversed(range(len(shape))))
+    strides, step = [], 1
+    for n in shape:
+        strides.append(step)
+        step *= max(n, 1)
+    return torch.empty_strided(shape, strides, dtype=tdt, device=device)
 
 
 def zeros(shape, dtype, order="F", device=None):
@@ -154,4 +163,4 @@ def ptr(t) -> int:
 
 def workspace(nbytes: int, device):
     """Scratch device memory from torch's caching allocator (current stream)."""
-    return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+    return torch.empty(int(nbytes) or 1, dtype=torch.uint8, device=device)

@@ -176,7 +176,13 @@ def call(name: str, *args) -> None:
     check(getattr(lib, name)(*args), name)
 
 
+_CODES = {"torch.float32": DTYPE_F32, "torch.float64": DTYPE_F64}
+
+
 def dtype_code(dtype) -> int:
+    code = _CODES.get(str(dtype))
+    if code is not None:
+        return code
     dtype = np.dtype(dtype) if not _is_torch_dtype(dtype) else _torch_to_np(dtype)
     if dtype == np.float32:
         return DTYPE_F32

@@ -21,8 +21,6 @@ Differences in kind, not in results:
 
 from __future__ import annotations
 
-import contextlib
-
 import numbers
 import sys
 from typing import Literal, TypeAlias
@@ -69,6 +67,8 @@ def _dims(arr):
 
 
 def _require_device_array(a, name):
+    if dev.is_device_array(a) and a.is_cuda:
+        return
     if not dev.is_device_array(a):
         raise TypeError(f"{name} must be a device array (torch.Tensor on a HIP device), got {type(a)}")
     if a.device.type != "cuda":
@@ -107,32 +107,43 @@ def launch_projection(is_fan, adjoint, out, inp, tables, img_shape, sinogram_sha
     and the operator API.  ``stream_is_current``: ``stream`` is torch's
     current stream of ``out``'s device, so the workspace is allocated there
     without switching streams (a few microseconds per call on small problems)."""
-    torch = dev.torch
+    _launch(is_fan, adjoint, out, inp, tables["ofs"], tables["geo"], tables["sdpd"] if is_fan else None,
+            img_shape, sinogram_shape, stream.cuda_stream, None if stream_is_current else stream)
+
+
+def _launch(is_fan, adjoint, out, inp, ofs, geo, sdpd, img_shape, sinogram_shape, handle, switch_to):
+    """launch_projection on the stream with this handle; ``switch_to`` is that
+    stream where it is not torch's current one, else None."""
     Nx, Ny = img_shape
     Ns, Na = sinogram_shape
     Nz = _dims(out)
-    in_order = dev.order_of(inp)
-    out_order = dev.order_of(out)
+    in_order = dev.order_code(dev.order_of(inp))
+    out_order = dev.order_code(dev.order_of(out))
     dcode = _hip.dtype_code(out.dtype)
-    geom = _hip.GEOM_FAN if is_fan else _hip.GEOM_RADON
     lib = _hip.load_library()
-    nbytes = lib.gt_projection_workspace_bytes(geom, int(adjoint), dcode, Nx, Ny, Ns, Na, Nz,
-                                               dev.order_code(in_order))
-    with contextlib.nullcontext() if stream_is_current else torch.cuda.stream(stream):
+    nbytes = lib.gt_projection_workspace_bytes(_hip.GEOM_FAN if is_fan else _hip.GEOM_RADON, int(adjoint), dcode,
+                                               Nx, Ny, Ns, Na, Nz, in_order)
+    if switch_to is None:
         ws = dev.workspace(nbytes, out.device)
-        head = (stream.cuda_stream, dcode, out.data_ptr(), inp.data_ptr(), tables["ofs"].data_ptr())
-        tail = (Nx, Ny, Ns, Na, Nz, dev.order_code(out_order), dev.order_code(in_order),
-                ws.data_ptr(), nbytes)
-        if is_fan:
-            name = "gt_fan_back" if adjoint else "gt_fan_fwd"
-            _hip.call(name, *head, tables["sdpd"].data_ptr(), tables["geo"].data_ptr(), *tail)
-        else:
-            name = "gt_radon_back" if adjoint else "gt_radon_fwd"
-            _hip.call(name, *head, tables["geo"].data_ptr(), *tail)
+    else:
+        with dev.torch.cuda.stream(switch_to):
+            ws = dev.workspace(nbytes, out.device)
+    if is_fan:
+        name, fn = ("gt_fan_back", lib.gt_fan_back) if adjoint else ("gt_fan_fwd", lib.gt_fan_fwd)
+        rc = fn(handle, dcode, out.data_ptr(), inp.data_ptr(), ofs.data_ptr(), sdpd.data_ptr(), geo.data_ptr(),
+                Nx, Ny, Ns, Na, Nz, out_order, in_order, ws.data_ptr(), nbytes)
+    else:
+        name, fn = ("gt_radon_back", lib.gt_radon_back) if adjoint else ("gt_radon_fwd", lib.gt_radon_fwd)
+        rc = fn(handle, dcode, out.data_ptr(), inp.data_ptr(), ofs.data_ptr(), geo.data_ptr(),
+                Nx, Ny, Ns, Na, Nz, out_order, in_order, ws.data_ptr(), nbytes)
+    if rc:
+        _hip.check(rc, name)
 
 
-def _project(out, inp, projectionsetting, adjoint, wait_for):
-    """Launch one projection: out = R inp (adjoint=False) or R^# inp."""
+def _project(out, inp, projectionsetting, adjoint, wait_for, record=True):
+    """Launch one projection: out = R inp (adjoint=False) or R^# inp.  Returns
+    an event recorded behind it (record=False: None; where nobody takes the
+    event, creating and recording it costs ~3 us of a small call's ~14)."""
     ps = projectionsetting
     if adjoint:
         img, sino = out, inp
@@ -143,14 +154,17 @@ def _project(out, inp, projectionsetting, adjoint, wait_for):
     check_compatibility(img, sino, ps)
     dtype = dev.to_np_dtype(sino.dtype)
     ps.ensure_dtype(dtype)
-    stream = _stream_of(ps)
-    _wait(stream, wait_for)
-    tables = {"ofs": ps.ofs_buf[dtype], "geo": ps.geometry_information[dtype]}
-    if ps.is_fan:
-        tables["sdpd"] = ps.sdpd_buf[dtype]
-    launch_projection(ps.is_fan, adjoint, out, inp, tables, ps.img_shape, ps.sinogram_shape, stream,
-                      stream_is_current=ps.queue.stream is None and out.device == ps.queue.device)
-    return _record(stream)
+    queue = ps.queue
+    # on torch's current stream of out's device nothing but its handle is needed
+    current = queue.stream is None and out.get_device() == queue.device.index
+    stream = None if current and not record and not wait_for else _stream_of(ps)
+    if wait_for:
+        _wait(stream, wait_for)
+    is_fan = ps.is_fan
+    _launch(is_fan, adjoint, out, inp, ps.ofs_buf[dtype], ps.geometry_information[dtype],
+            ps.sdpd_buf[dtype] if is_fan else None, ps.img_shape, ps.sinogram_shape,
+            queue.current_handle() if stream is None else stream.cuda_stream, None if current else stream)
+    return _record(stream) if record else None
 
 
 def forwardprojection(img, projectionsetting, sino=None, wait_for=[]):
@@ -544,16 +558,10 @@ class ProjectionSettings:
         self._geometry = GeometryType(value)
 
     def forwardprojection(self, sino, img, projectionsetting, wait_for=[]):
-        if self.geometry == GeometryType.RADON:
-            radon(sino, img, projectionsetting, wait_for=wait_for)
-        elif self.geometry == GeometryType.FANBEAM:
-            fanbeam(sino, img, projectionsetting, wait_for=wait_for)
+        _project(sino, img, projectionsetting, False, wait_for, record=False)
 
     def backprojection(self, img, sino, projectionsetting, wait_for=[]):
-        if self.geometry == GeometryType.RADON:
-            radon_ad(img, sino, projectionsetting, wait_for=wait_for)
-        elif self.geometry == GeometryType.FANBEAM:
-            fanbeam_ad(img, sino, projectionsetting, wait_for=wait_for)
+        _project(img, sino, projectionsetting, True, wait_for, record=False)
 
     def ensure_dtype(self, dtype):
         """Upload the tables of this dtype to the device once
