@@ -89,12 +89,8 @@ __global__ __launch_bounds__(256) void batch_relayout_kernel(const Job<real> *__
   const int4 t = tiles[blockIdx.x];
   const Job<real> J = load_job(jobs, t.x);
   const Strides3 ss = {1, J.Nx, (int64_t)J.Nx * J.Ny};
-  const Strides3 ys = {J.rowY, 1, J.sliceY};
-  relayout_tile(tile, const_cast<real *>(J.imgY), ys, J.src, ss, J.Nx, J.Ny, 0, t.y, t.z);
-  if (J.imgX != J.src) {
-    const Strides3 xs = {1, J.rowX, J.sliceX};
-    relayout_tile(tile, const_cast<real *>(J.imgX), xs, J.src, ss, J.Nx, J.Ny, 0, t.y, t.z);
-  }
+  relayout_pair(tile, J.imgX != J.src ? const_cast<real *>(J.imgX) : nullptr, J.rowX,
+                const_cast<real *>(J.imgY), J.rowY, J.src, ss, J.Nx, J.Ny, 0, t.y, t.z, 0);
 }
 
 // K = 1: tile (slice, bin block, angle block), 64 bins x 4 angles.  K > 1:
@@ -116,7 +112,7 @@ __global__ __launch_bounds__(256) void batch_fwd_kernel(const Job<real> *__restr
   } else {
     __shared__ real slots[Slots<K>::kCount * 256];
     int g;
-    const int a = group_lane<K>(t.y, J.Ns, J.Na, g);
+    const int a = group_lane<K>(t.y, J.Ns, J.Na, g, threadIdx.y);
     if (a >= J.Na) return;
     real *acc = slots + threadIdx.y * 64 + threadIdx.x;
     if (J.fan)
@@ -126,33 +122,38 @@ __global__ __launch_bounds__(256) void batch_fwd_kernel(const Job<real> *__restr
   }
 }
 
-// tile (slice, block of the slice's groups (group_lane), 0, band): one row
-// band of their strip walks; raw sums go to the slice's band partials
+// tile (slice, waves of the slice's groups, 0, set of bands), as fwd_band_kernel;
+// the sums of more than one set go to the slice's partials
 template <typename real, int K, int CH, int NB>
 __global__ __launch_bounds__(256) void batch_fwd_band_kernel(const Job<real> *__restrict__ jobs,
                                                              const int4 *__restrict__ tiles) {
+  constexpr int per = NB < kSubBands ? NB : kSubBands, sets = NB / per;
   __shared__ real slots[Slots<K>::kCount * 256];
   const int4 t = tiles[blockIdx.x];
   const Job<real> J = load_job(jobs, t.x);
+  const int w = t.y * (4 / per) + threadIdx.y / per, sub = threadIdx.y % per;
   int g;
-  const int a = group_lane<K>(t.y, J.Ns, J.Na, g);
-  if (a >= J.Na) return;
+  const int a = group_lane<K>(w >> 2, J.Ns, J.Na, g, w & 3);
   real *acc = slots + threadIdx.y * 64 + threadIdx.x;
-  const Band<real> B{t.w, NB, J.part};
-  if (J.fan)
-    fan_fwd_group<real, K, true, CH>(J, g * K, a, 0, acc, B);
-  else
-    radon_fwd_group<real, K, true, CH>(J, g * K, a, 0, acc, B);
+  const Band B{t.w * per + sub, NB};
+  if (a < J.Na) {
+    if (J.fan)
+      fan_fwd_group<real, K, true, CH>(J, g * K, a, 0, acc, B);
+    else
+      radon_fwd_group<real, K, true, CH>(J, g * K, a, 0, acc, B);
+  }
+  __syncthreads();
+  if (a < J.Na) subband_store<real, K>(J, J.part, t.w, sets, sub, per, g * K, a, 0, slots);
 }
 
-// tile (slice, angle): the bands of one sinogram row added in band order, then
-// the forward's scale and epilogue
-template <typename real, int NB>
+// tile (slice, angle): the band sets of one sinogram row added in order, then the
+// forward's scale and epilogue
+template <typename real, int SETS>
 __global__ __launch_bounds__(256) void batch_band_reduce_kernel(const Job<real> *__restrict__ jobs,
                                                                 const int4 *__restrict__ tiles) {
   const int4 t = tiles[blockIdx.x];
   const Job<real> J = load_job(jobs, t.x);
-  for (int s = threadIdx.x; s < J.Ns; s += 256) band_reduce_entry(J, J.part, NB, s, t.y, 0);
+  for (int s = threadIdx.x; s < J.Ns; s += 256) band_reduce_entry(J, J.part, SETS, s, t.y, 0);
 }
 
 // tile (slice, angle): one padded sinogram row
@@ -278,19 +279,21 @@ static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_ite
     if (chunked) X_at[i] = take(sizeof(real) * (size_t)(it.Nx + pad) * it.Ny);
   }
   const size_t copies_to = off;
-  if (nb > 1)
-    for (int i = 0; i < n; ++i) part_at[i] = take(sizeof(real) * (size_t)nb * items[i].Ns * items[i].Na);
+  if (nb > kSubBands)
+    for (int i = 0; i < n; ++i)
+      part_at[i] = take(sizeof(real) * (size_t)(nb / kSubBands) * items[i].Ns * items[i].Na);
   TileSet sets[5];
   for (int i = 0; i < n; ++i) {
     const gt_batch_item &it = items[i];
     // forward tile: ~ rows crossed x strip width per ray group
     const double cf =
         (double)std::max(it.Nx, it.Ny) * (K + 1) * (it.geometry == GT_GEOMETRY_FAN ? 1.5 : 1.0);
-    // bands innermost: the 8 bands of a tile are dispatched to the 8 XCDs in turn
-    if (K > 1) {  // blocks of 256 lanes over (angle, group) pairs (group_lane)
-      const int64_t nblk = group_blocks(it.Ns, it.Na, K);
+    // sets of bands innermost: they are dispatched to the 8 XCDs in turn
+    if (K > 1) {  // blocks of 256 lanes over (angle, group) pairs (group_lane) and a set's bands
+      const int64_t nblk = group_blocks(it.Ns, it.Na, K) * sub_bands(nb);
+      const int nset = nb / sub_bands(nb);
       for (int64_t b = 0; b < nblk; ++b)
-        for (int w = 0; w < nb; ++w) sets[kForward].add(i, (int)b, 0, cf / nb, w);
+        for (int w = 0; w < nset; ++w) sets[kForward].add(i, (int)b, 0, cf / nb, w);
     } else {  // 64 bins x 4 angles
       const int nsb = (it.Ns + 63) / 64, nab = (it.Na + 3) / 4;
       for (int b = 0; b < nsb; ++b)
@@ -347,7 +350,7 @@ static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_ite
     J.rowY = it.Ny + pad;
     J.sliceX = J.rowX * it.Ny;
     J.sliceY = J.rowY * it.Nx;
-    J.part = nb > 1 ? reinterpret_cast<real *>(base + part_at[i]) : nullptr;
+    J.part = nb > kSubBands ? reinterpret_cast<real *>(base + part_at[i]) : nullptr;
     J.io = order_strides(GT_ORDER_F, it.Nx, it.Ny, 1);
     J.S = reinterpret_cast<const real *>(base + S_at[i]);
     J.tab = reinterpret_cast<const AngleRec<real> *>(base + tab_at[i]);
@@ -436,20 +439,16 @@ static void launch_fwd_banded(const gt_batch_plan *p, hipStream_t st, const Job<
     case 8:
       hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, 8>), grid, block, 0, st, jobs,
                          p->tiles[kForward]);
-      hipLaunchKernelGGL((batch_band_reduce_kernel<real, 8>), dim3(p->n_tiles[kStage]), dim3(256), 0,
-                         st, jobs, p->tiles[kStage]);
+      hipLaunchKernelGGL((batch_band_reduce_kernel<real, 8 / kSubBands>), dim3(p->n_tiles[kStage]), dim3(256),
+                         0, st, jobs, p->tiles[kStage]);
       break;
     case 4:
       hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, 4>), grid, block, 0, st, jobs,
                          p->tiles[kForward]);
-      hipLaunchKernelGGL((batch_band_reduce_kernel<real, 4>), dim3(p->n_tiles[kStage]), dim3(256), 0,
-                         st, jobs, p->tiles[kStage]);
       break;
     default:
       hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, 2>), grid, block, 0, st, jobs,
                          p->tiles[kForward]);
-      hipLaunchKernelGGL((batch_band_reduce_kernel<real, 2>), dim3(p->n_tiles[kStage]), dim3(256), 0,
-                         st, jobs, p->tiles[kStage]);
   }
 }
 

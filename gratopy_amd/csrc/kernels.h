@@ -189,6 +189,32 @@ __device__ __forceinline__ void relayout_tile(real (*tile)[33], real *__restrict
   __syncthreads();
 }
 
+// One 32x32 block of both image copies of a strip walk, x-fastest rows of rowX
+// (first == nullptr: none) and y-fastest rows of rowY elements, read once; the
+// blocks at the end of a row also zero the `pad` elements behind it.
+template <typename real>
+__device__ __forceinline__ void relayout_pair(real (*tile)[33], real *__restrict__ cx, int64_t rowX,
+                                              real *__restrict__ cy, int64_t rowY,
+                                              const real *__restrict__ src, Strides3 ss, int Nx, int Ny,
+                                              int64_t z, int bx, int by, int pad) {
+  const bool x_first = ss.s0 <= ss.s1;
+  const int lx = threadIdx.x & 31, ly = threadIdx.x >> 5;
+  for (int k = ly; k < 32; k += 8) {
+    const int x = bx + (x_first ? lx : k), y = by + (x_first ? k : lx);
+    if (x < Nx && y < Ny) tile[x - bx][y - by] = src[x * ss.s0 + y * ss.s1 + z * ss.s2];
+  }
+  __syncthreads();
+  for (int k = ly; k < 32; k += 8) {
+    if (cx && bx + lx < Nx && by + k < Ny) cx[(z * Ny + by + k) * rowX + bx + lx] = tile[lx][k];
+    if (by + lx < Ny && bx + k < Nx) cy[(z * Nx + bx + k) * rowY + by + lx] = tile[k][lx];
+  }
+  for (int t = threadIdx.x; t < 32 * pad; t += 256) {
+    const int r = t / pad, f = t % pad;
+    if (cx && bx + 32 >= Nx && by + r < Ny) cx[(z * Ny + by + r) * rowX + Nx + f] = 0;
+    if (by + 32 >= Ny && bx + r < Nx) cy[(z * Nx + bx + r) * rowY + Ny + f] = 0;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Row ranges.  Conservative [ylo, yhi]: rows outside have no pixel in the
 // ray's strip (one row and one column of margin).
@@ -482,20 +508,23 @@ __device__ __forceinline__ void fan_fwd_ray(const Job<real> &J, int s, int a, in
 }
 
 // Row band of a banded forward launch: the strip walk is restricted to rows
-// [index*Nyy/count, (index+1)*Nyy/count) of its frame and the raw per-bin
-// sums go to part[((index*Nz + z)*Na + a)*Ns + s]; a second pass adds the
-// bands in order and applies the scale and epilogue (band_reduce_entry).
-template <typename real>
+// [index*Nyy/count, (index+1)*Nyy/count) of its frame and the raw per-bin sums
+// stay in the lane's slots 2 .. K + 1.  The sums of kSubBands (or, if fewer, all)
+// consecutive bands are added first, in band order, then those of the sets: in
+// the block that holds all bands of a set (subband_store) and from
+// part[((set*Nz + z)*Na + a)*Ns + s] (band_reduce_entry), or, in compacted
+// launches, from part[((index*Nz + z)*Na + a)*Ns + s].
 struct Band {
   int index, count;
-  real *part;
 };
 
-template <typename real>
-__device__ __forceinline__ real *band_slot(const Job<real> &J, const Band<real> &B, int s, int a,
-                                           int z) {
-  return B.part + (((int64_t)B.index * J.Nz + z) * J.Na + a) * J.Ns + s;
-}
+constexpr int kSubBands = 4;
+
+// Bands of at most this many rows are walked whole: passing by the rows that a
+// strip misses costs less than the four double divisions that clip them.
+constexpr int kShortBand = 24;
+
+__device__ __host__ __forceinline__ int sub_bands(int count) { return count < kSubBands ? count : kSubBands; }
 
 __device__ __forceinline__ void band_rows(int Nyy, int index, int count, int &ylo, int &yhi) {
   const int r0 = (int)((int64_t)Nyy * index / count);
@@ -509,17 +538,17 @@ __device__ __forceinline__ void band_rows(int Nyy, int index, int count, int &yl
 constexpr int kColumnAngles = 16;
 constexpr int kColumnGroups = 256 / kColumnAngles;
 
-// Lane of a whole-column block: wave y takes groups [4 y, 4 y + 4) of the
-// column for all 16 angles, lane x the angle x / 4 and group 4 y + x % 4.
+// Lane of a whole-column block: wave w takes groups [4 w, 4 w + 4) of the
+// column for all 16 angles, lane x the angle x / 4 and group 4 w + x % 4.
 // Returns the angle's index in the block; *goff the group's offset in the
 // column.  A wave then spans a few groups at 16 angles 0.25 degrees apart
 // (on the 1440-angle stacks): its lanes' strips have nearly equal widths
 // per row, so a row costs the wave little more than its lanes' own 16-byte
 // chunks (64 groups of one angle span ~40 % of a fan, whose strip widths
 // differ by a chunk or more), and its loads span a narrow part of the row.
-__device__ __forceinline__ int column_lane(int &goff) {
+__device__ __forceinline__ int column_lane(int &goff, int wave) {
   constexpr int LW = 64 / kColumnAngles;
-  goff = LW * threadIdx.y + (threadIdx.x % LW);
+  goff = LW * wave + (threadIdx.x % LW);
   return threadIdx.x / LW;
 }
 
@@ -534,7 +563,7 @@ __device__ __forceinline__ int column_lane(int &goff) {
 // holds the same detector edge for a run of adjacent angles.  Returns a (>=
 // Na for lanes past the end).
 template <int K>
-__device__ __forceinline__ int group_lane(int block, int Ns, int Na, int &g) {
+__device__ __forceinline__ int group_lane(int block, int Ns, int Na, int &g, int wave) {
   constexpr int A = kColumnAngles, C = kColumnGroups;
   const int groups = (Ns + K - 1) / K;
   const int cols = groups / C;
@@ -542,12 +571,12 @@ __device__ __forceinline__ int group_lane(int block, int Ns, int Na, int &g) {
   if (block < nfb) {
     const int ab = block / cols;
     int goff;
-    const int j = column_lane(goff);
+    const int j = column_lane(goff, wave);
     g = (block - ab * cols) * C + goff;
     return ab * A + j;
   }
   const int tail = groups - cols * C;
-  const int lin = (block - nfb) * 256 + threadIdx.y * 64 + threadIdx.x;
+  const int lin = (block - nfb) * 256 + wave * 64 + threadIdx.x;
   const int a = lin / tail;
   g = cols * C + (lin - a * tail);
   return a;
@@ -568,7 +597,7 @@ inline int64_t group_blocks(int Ns, int Na, int K) {
 // padding (the single-problem launches pad every row by 4 elements).
 template <typename real, int K, bool BANDED = false, int CH = 1, bool BUFW = false>
 __device__ __forceinline__ void fan_fwd_group(const Job<real> &J, int s0, int a, int z, real *acc,
-                                              Band<real> B = {}) {
+                                              Band B = {}) {
   using A = Arith<real>;
 #pragma unroll
   for (int k = 0; k < Slots<K>::kCount; ++k) acc[k * 256] = 0;
@@ -580,13 +609,14 @@ __device__ __forceinline__ void fan_fwd_group(const Job<real> &J, int s0, int a,
       if (!BANDED)
         fan_store(J, s, a, z, fan_ray_sum(J, s, a, z));
       else  // the ray's rows in this band, as for the regular groups
-        *band_slot(J, B, s, a, z) = fan_ray_sum(J, s, a, z, B.index, B.count);
+        acc[(k + 2) * 256] = fan_ray_sum(J, s, a, z, B.index, B.count);
     }
     return;
   }
-  int ylo, yhi;
-  fan_rows((double)F.qx, (double)F.qy, (double)F.dpx, (double)F.dmx, (double)F.midx,
-           (double)F.midy, F.Nxx, F.Nyy, ylo, yhi);
+  int ylo = 0, yhi = F.Nyy - 1;
+  if (!BANDED || F.Nyy > kShortBand * B.count)
+    fan_rows((double)F.qx, (double)F.qy, (double)F.dpx, (double)F.dmx, (double)F.midx,
+             (double)F.midy, F.Nxx, F.Nyy, ylo, yhi);
   if (BANDED) band_rows(F.Nyy, B.index, B.count, ylo, yhi);
   // Strip bounds in pixel columns: the bounding rays cross row y at
   // qx + midx + dpx (y - midy - qy) and qx + midx + dmx (y - midy - qy),
@@ -669,15 +699,11 @@ __device__ __forceinline__ void fan_fwd_group(const Job<real> &J, int s0, int a,
       } while (px <= end);
     }
   }
+  if (BANDED) return;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int s = s0 + k;
-    if (s >= J.Ns) continue;
-    const real sum = acc[(k + 2) * 256];
-    if (BANDED)
-      *band_slot(J, B, s, a, z) = sum;
-    else
-      fan_store(J, s, a, z, sum);
+    if (s < J.Ns) fan_store(J, s, a, z, acc[(k + 2) * 256]);
   }
 }
 
@@ -692,7 +718,7 @@ __device__ __forceinline__ real radon_scale(const Job<real> &J) {
 // CH: pixels per load along the strip row, as in fan_fwd_group.
 template <typename real, int K, bool BANDED = false, int CH = 1, bool BUFW = false>
 __device__ __forceinline__ void radon_fwd_group(const Job<real> &J, int s0, int a, int z,
-                                                real *acc, Band<real> B = {}) {
+                                                real *acc, Band B = {}) {
   using A = Arith<real>;
 #pragma unroll
   for (int k = 0; k < Slots<K>::kCount; ++k) acc[k * 256] = 0;
@@ -715,9 +741,10 @@ __device__ __forceinline__ void radon_fwd_group(const Job<real> &J, int s0, int 
     row_stride = J.rowX;
   }
   // union strip of the bins [s0, s0+K): centre s0 + (K-1)/2, half width (K+1)/2
-  int ylo, yhi;
-  radon_rows((double)X, (double)Y, (double)off - ((double)s0 + 0.5 * (K - 1)), 0.5 * (K + 1), Nxx,
-             Nyy, ylo, yhi);
+  int ylo = 0, yhi = Nyy - 1;
+  if (!BANDED || Nyy > kShortBand * B.count)
+    radon_rows((double)X, (double)Y, (double)off - ((double)s0 + 0.5 * (K - 1)), 0.5 * (K + 1), Nxx,
+               Nyy, ylo, yhi);
   if (BANDED) band_rows(Nyy, B.index, B.count, ylo, yhi);
   const real lo = (real)0.5, hi = (real)K + (real)2.5;
   // the strip's rays through s0 - 1 and s0 + K, ordered by the column they
@@ -782,21 +809,47 @@ __device__ __forceinline__ void radon_fwd_group(const Job<real> &J, int s0, int 
       } while (px <= end);
     }
   }
+  if (BANDED) return;
   const real scale = radon_scale(J);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int s = s0 + k;
-    if (s >= J.Ns) continue;
-    const real sum = acc[(k + 2) * 256];
-    if (BANDED)
-      *band_slot(J, B, s, a, z) = sum;
-    else
-      store_fwd(J, s, a, z, sum * scale);
+    if (s < J.Ns) store_fwd(J, s, a, z, acc[(k + 2) * 256] * scale);
   }
 }
 
-// Sum of the row bands of bin (s, a, z) in band order, then the per-ray scale
-// and epilogue of the unbanded bodies.
+// A finished sum: the per-ray scale and epilogue.
+template <typename real>
+__device__ __forceinline__ void sum_store(const Job<real> &J, int s, int a, int z, real sum) {
+  if (J.fan)
+    fan_store(J, s, a, z, sum);
+  else
+    store_fwd(J, s, a, z, sum * radon_scale(J));
+}
+
+// A banded block whose waves hold the kSubBands (or all count) bands of set
+// `set` for the same lanes (`per` waves, this one band `sub` of them): adds them
+// in band order; the bins are split over the waves.
+template <typename real, int K>
+__device__ __forceinline__ void subband_store(const Job<real> &J, real *part, int set, int sets, int sub, int per,
+                                              int s0, int a, int z, const real *slots) {
+  const real *acc = slots + (threadIdx.y - sub) * 64 + threadIdx.x;
+#pragma unroll 1
+  for (int k = sub; k < K; k += per) {
+    const int s = s0 + k;
+    if (s >= J.Ns) break;
+    real sum = acc[(k + 2) * 256];
+    for (int j = 1; j < per; ++j) sum += acc[(k + 2) * 256 + 64 * j];
+    if (sets == 1)
+      sum_store(J, s, a, z, sum);
+    else
+      part[(((int64_t)set * J.Nz + z) * J.Na + a) * J.Ns + s] = sum;
+  }
+}
+
+// Sum of the row bands of bin (s, a, z), sets first, then the per-ray scale and
+// epilogue of the unbanded bodies.  part holds the sums of `count` sets, or, with
+// range, of a compacted launch's `count` bands.
 template <typename real>
 __device__ __forceinline__ void band_reduce_entry(const Job<real> &J, const real *__restrict__ part,
                                                   int count, int s, int a, int z,
@@ -809,24 +862,23 @@ __device__ __forceinline__ void band_reduce_entry(const Job<real> &J, const real
     // others are exact zeros there (no strip pixel in the band), added as
     // such so that the sum is the uncompacted one bit for bit
     const int g = s / K;
+    const int per = sub_bands(count);
     real acc = 0;
-    for (int b = 0; b < count; ++b) {
-      const int2 r = range[(int64_t)b * J.Na + a];
-      const real v = (g >= r.x && g < r.y) ? p[b * stride] : (real)0;
-      acc = b == 0 ? v : acc + v;
+    for (int b = 0; b < count; b += per) {
+      real set = 0;
+      for (int j = 0; j < per; ++j) {
+        const int2 r = range[(int64_t)(b + j) * J.Na + a];
+        const real v = (g >= r.x && g < r.y) ? p[(b + j) * stride] : (real)0;
+        set = j == 0 ? v : set + v;
+      }
+      acc = b == 0 ? set : acc + set;
     }
-    if (J.fan)
-      fan_store(J, s, a, z, acc);
-    else
-      store_fwd(J, s, a, z, acc * radon_scale(J));
+    sum_store(J, s, a, z, acc);
     return;
   }
   real acc = p[0];
   for (int b = 1; b < count; ++b) acc += p[b * stride];
-  if (J.fan)
-    fan_store(J, s, a, z, acc);
-  else
-    store_fwd(J, s, a, z, acc * radon_scale(J));
+  sum_store(J, s, a, z, acc);
 }
 
 // ---------------------------------------------------------------------------

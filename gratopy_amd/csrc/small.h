@@ -78,7 +78,7 @@ __device__ __forceinline__ void fwd_small_block(const Job<real> &J, Strides3 ii,
       // The window of the next rows: the edge rays are the extremes and linear
       // along the rows; one whole column to spare on each side for the rounding.
       FwdChunk c{y, min(kSmallRows, y1 - y), 0, 0, 0};
-      double lo = 1e30, hi = -1e30, w = 0, xl = 1e30, xr = -1e30;
+      double lo = 1e30, hi = -1e30, w = 0, xr = -1e30;
       for (int end = 0; end < 2; ++end) {
         const double ye = end ? y + c.rows - 1 : y;
         const double ua = fma(m0, ye, u0), ub = fma(m1, ye, u1), va = fma(n0, ye, v0), vb = fma(n1, ye, v1);
