@@ -340,11 +340,11 @@ struct FanStrip {
   int Nxx, Nyy;
   const real *base;
   int64_t row_stride;
-  // both bounding rays advance the same way along the row axis, so each row
-  // meets the strip in one interval [xlow(y), xhigh(y)].  The rays of a
-  // single bin always do on the reference's geometries; the union strip of a
-  // bin group can fail it when bins are very wide (a few detector bins over
-  // a large angle), and the group then projects its bins one by one.
+  // both bounding rays run from the source to the rows on the image's side (for
+  // which left and right are told apart), so each row meets the strip in one
+  // interval [xlow(y), xhigh(y)].  The rays of a single bin always do on the
+  // reference's geometries; the union strip of a bin group can fail it in wide
+  // fans or with very wide bins, and the group then projects its bins one by one.
   bool regular;
 };
 
@@ -392,7 +392,7 @@ __device__ __forceinline__ FanStrip<real> fan_strip(const Job<real> &J, int a, i
     F.base = J.imgY + z * J.sliceY;
     F.row_stride = J.rowY;
   }
-  F.regular = dpy * dmy > (real)0;
+  F.regular = qy * dpy < (real)0 && qy * dmy < (real)0;
   dpx /= dpy;
   dmx /= dmy;
   if (qy * (dmx - dpx) < (real)0) {
@@ -636,7 +636,9 @@ __device__ __forceinline__ void fan_fwd_group(const Job<real> &J, int s0, int a,
   const double c0 = (double)J.geo[5] - (double)s0 + 2.0;
   const double tdx = F.ddx, tdy = F.ddy;
   const double qdx = (double)F.dx + c0 * tdx, qdy = (double)F.dy + c0 * tdy;
-  const real dq = (real)qdx;
+  real ts[CH + 1], qs[CH + 1];
+#pragma unroll
+  for (int i = 1; i <= CH; ++i) ts[i] = (real)i * F.ddx, qs[i] = (real)i * (real)qdx;
   const real lo = (real)0.5, hi = (real)K + (real)2.5;
   const double ud0 = (double)ylo - (double)F.midy;
   const real t00 = (real)(tdy * ud0 + (double)F.RE - tdx * (double)F.midx);
@@ -659,15 +661,16 @@ __device__ __forceinline__ void fan_fwd_group(const Job<real> &J, int s0, int a,
     const int dy = y - ylo;
     real t = fma(F.ddx, (real)xl, fma(F.ddy, (real)dy, t00));
     real q = (real)fma(qdx, (double)xl, fma(qdy, (double)dy, q00));
+    // one rounding per chunk in the running t and q: pixel i is i steps from them
     auto chunk = [&](const RowChunk<real, CH> &c) {
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
-        const real r = A::rcp(t);
-        const real p = A::clamp(q * r, lo, hi);
+        const real r = A::rcp(i == 0 ? t : t + ts[i]);
+        const real p = A::clamp((i == 0 ? q : q + qs[i]) * r, lo, hi);
         deposit(acc, p, c.v[i] * r);
-        t += F.ddx;
-        q += dq;
       }
+      t += ts[CH];
+      q += qs[CH];
     };
     if constexpr (BUFW) {
       const int end = roff + xh * (int)sizeof(real);
@@ -751,6 +754,9 @@ __device__ __forceinline__ void radon_fwd_group(const Job<real> &J, int s0, int 
   // reach first along a row (inv = 1/X carries the direction)
   const real s_first = inv < (real)0 ? (real)(s0 + K) : (real)(s0 - 1);
   const real s_last = inv < (real)0 ? (real)(s0 - 1) : (real)(s0 + K);
+  real xs[CH + 1];
+#pragma unroll
+  for (int i = 1; i <= CH; ++i) xs[i] = (real)i * X;
   const double p00 = (double)off - (double)s0 + 2.0;  // pixel (0, 0) relative to bin s0 - 2
   // row y starts at base + y * row_stride, walked by one add per row
   const real *row = base + (int64_t)ylo * row_stride;
@@ -773,12 +779,11 @@ __device__ __forceinline__ void radon_fwd_group(const Job<real> &J, int s0, int 
     // evaluated in double: x*X and y*Y + off are up to Ns in size and nearly
     // cancel; inside the strip it lies in [1, K+2], so truncation is floor
     real pr = (real)fma((double)X, (double)xl, fma((double)Y, (double)y, p00));
+    // one rounding per chunk in the running position: pixel i is i steps from it
     auto chunk = [&](const RowChunk<real, CH> &c) {
 #pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        deposit(acc, A::clamp(pr, lo, hi), c.v[i]);
-        pr += X;
-      }
+      for (int i = 0; i < CH; ++i) deposit(acc, A::clamp(i == 0 ? pr : pr + xs[i], lo, hi), c.v[i]);
+      pr += xs[CH];
     };
     if constexpr (BUFW) {
       const int end = roff + xh * (int)sizeof(real);

@@ -821,6 +821,54 @@ static size_t fwd_ws(int dtype, const Layout &L, int img_order) {
   return n;
 }
 
+// Calls that take less time than the launches of the paths above go in one
+// launch (small.h), without the workspace those need (its size is still checked).
+// Microseconds on the GPU, before -> after.  Forward: 64^2, 44 angles, 89
+// detectors 17.8 -> 5.7; 128^2, 89 angles 24.5 -> 9.5 (fan 24.0 -> 14.1); 192^2,
+// 130 angles 35 -> 17 (fan 32 -> 24); 256^2, 179 angles (not taken) 32.4 against
+// 31.6, in C order 32.6 against 36.0.  Back: 64^2 21 -> 4.0 (fan 21.8 -> 5.8);
+// 128^2 38.5 -> 5.2 (fan 40.4 -> 6.8); 256^2 16.8 -> 8.1 (fan 18.0 -> 12.8,
+// float64 21.5 -> 17.0); 400^2, 280 angles float32 parallel beam 31.8 -> 22.6
+// (not taken: float64 34.8 against 38.3, fan 33.4 against 51.3).
+static bool fwd_is_small(const Layout &L) {
+  return tuning().automatic && work_of(L) < 8e6;
+}
+
+static bool back_is_small(int dtype, const Layout &L) {
+  return tuning().automatic && work_of(L) < (L.fan || dtype == GT_FLOAT64 ? 2e7 : 5e7);
+}
+
+// Automatic forward calls of single slices (and what the slice-batched forward
+// leaves): the banded 16-byte reads, with more bands than the shapes above since
+// only every kSubBands-th band costs a partial sum, and without compaction, whose
+// lists cannot keep a set's bands together.  Taken where the workspace holds it;
+// a smaller one gets the shapes above.  GPU us with 16 / 32 / 48 / 64 bands of K =
+// 8 and 16 bins a lane (before: the shapes above):
+//   fan 256^2, 180 angles        8: 27.4 / 24.3 / 25.1 / 26.5, 16: - / 26.4 / 27.2 / 26.4  (44.9)
+//   fan 384^2, 240 angles        8: 46.7 / 39.2 / 41.2 / 43.4, 16: - / 41.8 / 42.4 / 40.1  (69.4)
+//   fan 512^2, 360 angles        8: 84.9 / 75.7 / 80.2 / 84.7, 16: 88.6 / 71.5 / 71.2 / 72.0  (75.8)
+//   parallel 512^2, 360 angles   8: - / 70.0 / 69.2 / 70.5, 16: 80.3 / 75.5 / 74.8 / 73.3  (70.1)
+//   parallel 1024^2, 720 angles  8: 369 / 355 / 353 / 358, 16: 375 / 350 / 332 / 341  (354)
+//   fan 1024^2, 720 angles       8: 412 / 416 / 411 / -, 16: 365 / 346 / 336 / 360  (415)
+//   parallel 2048^2, 1440 angles 16: 2321 / 2204 / 2211 / 2194  (2307)
+//   fan 2048^2, 1440 angles      16: 2282 / 2223 / 2167 / 2376  (2491)
+// 48 bands of fewer than 10 rows lose to 32, and launches that fill the GPU many
+// times over take 16, for the memory of the sums.  16 bins a lane need enough lanes:
+// 2048 blocks are as many as the GPU holds (2 x 600^2 fan, 120 angles, 328
+// detectors, 48 bands: 76.1 us with 8, 78.0 with 16).
+static FwdShape fwd_run_shape(const Layout &L) {
+  const int64_t blocks = group_blocks(L.Ns, L.Na, 16) * L.Nz, rows = std::min(L.Nx, L.Ny);
+  const int bands = rows < 200 || blocks > 2500 ? 16 : rows < 480 ? 32 : 48;
+  const int K = work_of(L) < (L.fan ? 6e7 : 2e8) || blocks * bands < 2048 ? 8 : 16;
+  return {K, bands, 4, false};
+}
+
+static size_t fwd_run_ws(int dtype, const Layout &L) {
+  const size_t e = elem_size(dtype);
+  return align_up(e * (size_t)(L.Nx + kRowPad) * L.Ny * L.Nz) + align_up(e * (size_t)(L.Ny + kRowPad) * L.Nx * L.Nz) +
+         align_up(e * (size_t)(fwd_run_shape(L).bands / kSubBands) * L.Ns * L.Na * L.Nz);
+}
+
 static size_t back_partials(int dtype, const Layout &L) {
   const int nb = back_shape(L).bands;
   return nb > 1 ? align_up(elem_size(dtype) * (size_t)nb * L.Nx * L.Ny * L.Nz) : 0;
@@ -937,24 +985,9 @@ static size_t fwd_stack_ws(int dtype, const Layout &L, const FwdStackShape &s) {
 
 static size_t fwd_need(int dtype, const Layout &L, int img_order) {
   const FwdStackShape s = fwd_stack_shape(dtype, L);
-  return s.g ? fwd_stack_ws(dtype, L, s) : fwd_ws(dtype, L, img_order);
-}
-
-// Calls that take less time than the launches of the paths above go in one
-// launch (small.h), without the workspace those need (its size is still checked).
-// Microseconds on the GPU, before -> after.  Forward: 64^2, 44 angles, 89
-// detectors 17.8 -> 5.7; 128^2, 89 angles 24.5 -> 9.5 (fan 24.0 -> 14.1); 192^2,
-// 130 angles 35 -> 17 (fan 32 -> 24); 256^2, 179 angles (not taken) 32.4 against
-// 31.6, in C order 32.6 against 36.0.  Back: 64^2 21 -> 4.0 (fan 21.8 -> 5.8);
-// 128^2 38.5 -> 5.2 (fan 40.4 -> 6.8); 256^2 16.8 -> 8.1 (fan 18.0 -> 12.8,
-// float64 21.5 -> 17.0); 400^2, 280 angles float32 parallel beam 31.8 -> 22.6
-// (not taken: float64 34.8 against 38.3, fan 33.4 against 51.3).
-static bool fwd_is_small(const Layout &L) {
-  return tuning().automatic && work_of(L) < 8e6;
-}
-
-static bool back_is_small(int dtype, const Layout &L) {
-  return tuning().automatic && work_of(L) < (L.fan || dtype == GT_FLOAT64 ? 2e7 : 5e7);
+  if (s.g) return fwd_stack_ws(dtype, L, s);
+  const size_t need = fwd_ws(dtype, L, img_order);
+  return tuning().automatic && !fwd_is_small(L) ? std::max(need, fwd_run_ws(dtype, L)) : need;
 }
 
 template <typename real>
@@ -1075,7 +1108,7 @@ static int fwd_impl(hipStream_t st, real *sino, const real *img, const real *ofs
   if (ss.g && ws != nullptr && ws_bytes >= fwd_stack_ws(dtype, L, ss))
     return fwd_stack_impl<real, FAN>(st, sino, img, ofs, sdpd, geo, L, sino_order, img_order,
                                      static_cast<char *>(ws), ss);
-  const size_t need = fwd_ws(dtype, L, img_order);
+  size_t need = fwd_ws(dtype, L, img_order);
   if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
   GT_REQUIRE(need == 0 || ws != nullptr, "workspace pointer is NULL");
   const Strides3 is = order_strides(img_order, L.Nx, L.Ny, L.Nz);
@@ -1094,12 +1127,18 @@ static int fwd_impl(hipStream_t st, real *sino, const real *img, const real *ofs
       hipLaunchKernelGGL((fwd_small_kernel<real, FAN, 8, 1024>), grid, dim3(512), 0, st, J, is);
     return check_launch(FAN ? "fan forward projection" : "radon forward projection");
   }
+  FwdShape sh = fwd_shape(L);
+  int parts = sh.bands;  // partial sums in the workspace
+  if (tuning().automatic && ws != nullptr && ws_bytes >= fwd_run_ws(dtype, L)) {
+    sh = fwd_run_shape(L);
+    parts = sh.bands / kSubBands;
+    need = fwd_run_ws(dtype, L);
+  }
   J.imgX = img;
   J.imgY = img;
   J.rowX = L.Nx;
   J.rowY = L.Ny;
   J.sliceX = J.sliceY = (int64_t)L.Nx * L.Ny;
-  const FwdShape sh = fwd_shape(L);
   if (sh.chunk > 1) {
     const int64_t rx = L.Nx + kRowPad, ry = L.Ny + kRowPad;
     real *cx = reinterpret_cast<real *>(w);
@@ -1142,7 +1181,7 @@ static int fwd_impl(hipStream_t st, real *sino, const real *img, const real *ofs
   if (nb > 1) {
     // the band partials are the last part of the workspace, the group plan
     // (compacted launches) comes before them, after the image copies
-    const size_t part_bytes = align_up(sizeof(real) * (size_t)nb * L.Ns * L.Na * L.Nz);
+    const size_t part_bytes = align_up(sizeof(real) * (size_t)parts * L.Ns * L.Na * L.Nz);
     part = reinterpret_cast<real *>(static_cast<char *>(ws) + (need - part_bytes));
     if (sh.compact) {
       int2 *q = reinterpret_cast<int2 *>(static_cast<char *>(ws) + (need - part_bytes -

@@ -1,0 +1,69 @@
+"""The automatic banded forward against the oracle: both group widths and every
+band count, thin images whose bands hold a row or none, single bins and part
+groups, two slices, wide fans whose groups leave their frame, and a workspace
+that holds only the launch shape of the workspace-free entry point."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import gratopy_amd as gratopy
+from gratopy_amd import _device as dev
+from gratopy_amd import _hip, autotune
+from tests.helpers import rel_err
+from tests.test_gpu_projection import TOL, _oracle
+from tests.test_gpu_stack_fwd import _settings
+
+pytestmark = pytest.mark.gpu
+
+F32, F64 = np.dtype("float32"), np.dtype("float64")
+
+# (geometry, image, slices, angles, detectors, dtype, order, further settings);
+# single slices of at least 8e6 pixel-angles
+CALLS = [
+    ("radon", (199, 210), 1, 200, 300, F32, "F", {}),    # 16 bands
+    ("radon", (201, 200), 1, 201, 17, F32, "C", {}),     # 32; a bin over a pair of groups
+    ("fan", (479, 480), 1, 60, 500, F64, "F", {}),       # 32 bands, 8 bins
+    ("fan", (481, 480), 1, 300, 512, F32, "C", {}),      # 48 bands, 16 bins
+    ("radon", (480, 500), 1, 900, 513, F32, "F", {}),
+    ("radon", (20, 2000), 1, 250, 600, F64, "F", {}),    # bands of one row or two
+    ("fan", (3000, 9), 1, 320, 700, F32, "F", {}),       # empty bands
+    ("fan", (300, 290), 2, 400, 1, F32, "C", {}),        # a single bin
+    ("radon", (256, 256), 2, 200, 391, F32, "F", {}),
+    ("fan", (230, 230), 1, 170, 345, F32, "F", dict(detector_width=1840.0)),  # half angle 63 degrees
+    ("fan", (300, 300), 1, 100, 100, F64, "F", dict(detector_width=9000.0)),  # 82 degrees
+]
+
+
+@pytest.mark.parametrize("geometry,shape,nz,angles,nd,dtype,order,more", CALLS)
+def test_banded_forward_against_the_oracle(geometry, shape, nz, angles, nd, dtype, order, more):
+    print(f"banded forward {geometry} {shape} x {nz}, {angles} angles, {nd} det, {dtype}, {order}, {more}", flush=True)
+    before = autotune.current_variant()
+    try:
+        autotune.set_variant(automatic=1)
+        ps = _settings(geometry, shape, angles, nd, more)
+        z = (nz,) if nz > 1 else ()
+        img = np.require(np.random.default_rng(43).random(shape + z).astype(dtype), requirements=order)
+        d_img = dev.to_device(img, "cuda:0", order=order)
+        got = dev.to_host(gratopy.forwardprojection(d_img, ps)).reshape(nd, angles, nz)
+        # the entry point without allocations, and one that was given no more than
+        # its shape needs, take either route
+        small = dev.zeros((nd, angles) + z, dtype, order="F", device="cuda:0")
+        tables = [ps.ofs_buf[dtype], ps.sdpd_buf[dtype] if ps.is_fan else None, ps.geometry_information[dtype]]
+        _hip.call("gt_projection_noalloc", torch.cuda.current_stream().cuda_stream, int(ps.is_fan), 0,
+                  _hip.dtype_code(dtype), small.data_ptr(), d_img.data_ptr(),
+                  tables[0].data_ptr(), tables[1].data_ptr() if ps.is_fan else None, tables[2].data_ptr(),
+                  *shape, nd, angles, nz, 0, dev.order_code(order))
+        torch.cuda.synchronize()
+        for result in (got, dev.to_host(small).reshape(nd, angles, nz)):
+            for k in range(nz):
+                x = img.reshape(shape + (nz,))[:, :, k]
+                ref = _oracle(ps, x.astype(F64), F64, False)
+                bar = TOL[dtype]
+                if dtype == F32:
+                    bar = max(bar, 1.2 * rel_err(_oracle(ps, x, F32, False), ref))
+                assert rel_err(result[:, :, k], ref) <= bar, k
+    finally:
+        autotune.set_variant(**before)
