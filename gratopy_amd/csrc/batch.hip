@@ -28,7 +28,9 @@ struct gt_batch_plan {
   int dtype;
   int n_items;
   int fwd_group, back_rows;
-  int fwd_bands;              // > 1: row-banded forward (per-slice partials, ordered reduction)
+  bool fwd_banded;            // row-banded forward
+  bool fwd_partials;          // with partial sums in memory and an ordered reduction
+  bool fwd_bufw;              // strip walks by buffer offsets
   int fwd_chunk;              // 4: forward strip rows read from row-padded copies, 16 bytes per load
   int back_stage, back_tile;  // > 0: LDS-staged backprojection (angles per chunk, tile width)
   bool has_data;  // every item has data (Landweber, TV)
@@ -124,36 +126,37 @@ __global__ __launch_bounds__(256) void batch_fwd_kernel(const Job<real> *__restr
 
 // tile (slice, waves of the slice's groups, 0, set of bands), as fwd_band_kernel;
 // the sums of more than one set go to the slice's partials
-template <typename real, int K, int CH, int NB>
+template <typename real, int K, int CH, bool BUFW>
 __global__ __launch_bounds__(256) void batch_fwd_band_kernel(const Job<real> *__restrict__ jobs,
                                                              const int4 *__restrict__ tiles) {
-  constexpr int per = NB < kSubBands ? NB : kSubBands, sets = NB / per;
   __shared__ real slots[Slots<K>::kCount * 256];
   const int4 t = tiles[blockIdx.x];
   const Job<real> J = load_job(jobs, t.x);
+  const int per = sub_bands(J.bands);
   const int w = t.y * (4 / per) + threadIdx.y / per, sub = threadIdx.y % per;
   int g;
   const int a = group_lane<K>(w >> 2, J.Ns, J.Na, g, w & 3);
   real *acc = slots + threadIdx.y * 64 + threadIdx.x;
-  const Band B{t.w * per + sub, NB};
+  const Band B{t.w * per + sub, J.bands};
   if (a < J.Na) {
     if (J.fan)
-      fan_fwd_group<real, K, true, CH>(J, g * K, a, 0, acc, B);
+      fan_fwd_group<real, K, true, CH, BUFW>(J, g * K, a, 0, acc, B);
     else
-      radon_fwd_group<real, K, true, CH>(J, g * K, a, 0, acc, B);
+      radon_fwd_group<real, K, true, CH, BUFW>(J, g * K, a, 0, acc, B);
   }
   __syncthreads();
-  if (a < J.Na) subband_store<real, K>(J, J.part, t.w, sets, sub, per, g * K, a, 0, slots);
+  if (a < J.Na) subband_store<real, K>(J, J.part, t.w, J.bands / per, sub, per, g * K, a, 0, slots);
 }
 
 // tile (slice, angle): the band sets of one sinogram row added in order, then the
 // forward's scale and epilogue
-template <typename real, int SETS>
+template <typename real>
 __global__ __launch_bounds__(256) void batch_band_reduce_kernel(const Job<real> *__restrict__ jobs,
                                                                 const int4 *__restrict__ tiles) {
   const int4 t = tiles[blockIdx.x];
   const Job<real> J = load_job(jobs, t.x);
-  for (int s = threadIdx.x; s < J.Ns; s += 256) band_reduce_entry(J, J.part, SETS, s, t.y, 0);
+  if (J.bands <= kSubBands) return;
+  for (int s = threadIdx.x; s < J.Ns; s += 256) band_reduce_entry(J, J.part, J.bands / kSubBands, s, t.y, 0);
 }
 
 // tile (slice, angle): one padded sinogram row
@@ -233,20 +236,25 @@ static int check_item(const gt_batch_item &it) {
   return GT_OK;
 }
 
+// The tiles of one launch kind, all of a slice at one cost.
 struct TileSet {
   std::vector<int4> t;
-  std::vector<double> cost;
-  void add(int item, int a, int b, double c, int w = 0) {
-    t.push_back(make_int4(item, a, b, w));
+  std::vector<size_t> from;  // first tile of each slice
+  std::vector<double> cost;  // of each slice's tiles
+  void item(double c) {
+    from.push_back(t.size());
     cost.push_back(c);
   }
+  void add(int a, int b, int w = 0) { t.push_back(make_int4((int)from.size() - 1, a, b, w)); }
   // largest first; ties keep slice order
   std::vector<int4> sorted() const {
-    std::vector<size_t> idx(t.size());
+    std::vector<size_t> idx(from.size());
     for (size_t i = 0; i < idx.size(); ++i) idx[i] = i;
     std::stable_sort(idx.begin(), idx.end(), [&](size_t a, size_t b) { return cost[a] > cost[b]; });
-    std::vector<int4> out(t.size());
-    for (size_t i = 0; i < idx.size(); ++i) out[i] = t[idx[i]];
+    std::vector<int4> out;
+    out.reserve(t.size());
+    for (size_t i : idx)
+      out.insert(out.end(), t.begin() + from[i], i + 1 < from.size() ? t.begin() + from[i + 1] : t.end());
     return out;
   }
 };
@@ -256,9 +264,21 @@ constexpr int kBatchRowPad = 4;
 
 template <typename real>
 static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_item *items, int K,
-                       int RY, int nb, int chunk, int stage, int tx) {
+                       int RY, int fwd_bands, int chunk, int stage, int tx) {
   const bool chunked = K > 1 && chunk > 1;
-  nb = K > 1 && nb > 1 ? nb : 1;
+  // Row bands of each slice: fwd_bands, or (0) by its rows and the blocks of the
+  // batch, much as the single-slice forward chooses them (16 slices of 256^2 ..
+  // 1024^2, 5 iterations: 8.33 ms with 8 bands, 7.47 with at most 32, 7.60 with
+  // 48; 64 slices, 20 iterations: 108 ms with 8, 100 with 16, 104 with 32).
+  std::vector<int> bands(n, K > 1 && fwd_bands > 1 ? fwd_bands : 1);
+  if (fwd_bands == 0) {
+    int64_t blocks = 0;
+    for (int i = 0; i < n; ++i) blocks += group_blocks(items[i].Ns, items[i].Na, K);
+    for (int i = 0; i < n; ++i) {
+      const int rows = std::min(items[i].Nx, items[i].Ny);
+      bands[i] = rows < 200 || blocks > 2500 ? 16 : 32;
+    }
+  }
   const int pad = chunked ? kBatchRowPad : 0;
   const int ty = 256 / tx;  // lane rows of a staged tile
   // ---- layout of the single allocation ----
@@ -271,43 +291,53 @@ static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_ite
   const size_t jobs_at = take(4 * sizeof(Job<real>) * (size_t)n);
   std::vector<size_t> tab_at(n), S_at(n), Y_at(n), X_at(n), part_at(n);
   const size_t copies_from = off;
+  bool bufw = chunked;  // every slice's two copies lie within one descriptor's reach
   for (int i = 0; i < n; ++i) {
     const gt_batch_item &it = items[i];
     tab_at[i] = take(sizeof(AngleRec<real>) * (size_t)it.Na);
     S_at[i] = take(sizeof(real) * (size_t)(it.Ns + 4) * it.Na);
-    Y_at[i] = take(sizeof(real) * (size_t)(it.Ny + pad) * it.Nx);
     if (chunked) X_at[i] = take(sizeof(real) * (size_t)(it.Nx + pad) * it.Ny);
+    Y_at[i] = take(sizeof(real) * (size_t)(it.Ny + pad) * it.Nx);
+    bufw = bufw && strip_buffer_fits(off - X_at[i]);
   }
   const size_t copies_to = off;
-  if (nb > kSubBands)
-    for (int i = 0; i < n; ++i)
-      part_at[i] = take(sizeof(real) * (size_t)(nb / kSubBands) * items[i].Ns * items[i].Na);
+  bool partials = false;
+  for (int i = 0; i < n; ++i)
+    if (bands[i] > kSubBands) {
+      partials = true;
+      part_at[i] = take(sizeof(real) * (size_t)(bands[i] / kSubBands) * items[i].Ns * items[i].Na);
+    }
   TileSet sets[5];
   for (int i = 0; i < n; ++i) {
     const gt_batch_item &it = items[i];
+    const int nb = bands[i];
     // forward tile: ~ rows crossed x strip width per ray group
     const double cf =
         (double)std::max(it.Nx, it.Ny) * (K + 1) * (it.geometry == GT_GEOMETRY_FAN ? 1.5 : 1.0);
     // sets of bands innermost: they are dispatched to the 8 XCDs in turn
+    sets[kForward].item(cf / nb);
     if (K > 1) {  // blocks of 256 lanes over (angle, group) pairs (group_lane) and a set's bands
       const int64_t nblk = group_blocks(it.Ns, it.Na, K) * sub_bands(nb);
       const int nset = nb / sub_bands(nb);
       for (int64_t b = 0; b < nblk; ++b)
-        for (int w = 0; w < nset; ++w) sets[kForward].add(i, (int)b, 0, cf / nb, w);
+        for (int w = 0; w < nset; ++w) sets[kForward].add((int)b, 0, w);
     } else {  // 64 bins x 4 angles
       const int nsb = (it.Ns + 63) / 64, nab = (it.Na + 3) / 4;
       for (int b = 0; b < nsb; ++b)
-        for (int a = 0; a < nab; ++a) sets[kForward].add(i, b, a, cf);
+        for (int a = 0; a < nab; ++a) sets[kForward].add(b, a);
     }
+    sets[kRelayout].item(1.0);
     for (int bx = 0; bx < (it.Nx + 31) / 32; ++bx)
-      for (int by = 0; by < (it.Ny + 31) / 32; ++by) sets[kRelayout].add(i, bx * 32, by * 32, 1.0);
-    for (int a = 0; a < it.Na; ++a) sets[kStage].add(i, a, 0, (double)it.Ns);
-    const double cb = (double)it.Na * RY * (it.geometry == GT_GEOMETRY_FAN ? 1.5 : 1.0);
+      for (int by = 0; by < (it.Ny + 31) / 32; ++by) sets[kRelayout].add(bx * 32, by * 32);
+    sets[kStage].item((double)it.Ns);
+    for (int a = 0; a < it.Na; ++a) sets[kStage].add(a, 0);
+    sets[kBackward].item((double)it.Na * RY * (it.geometry == GT_GEOMETRY_FAN ? 1.5 : 1.0));
     const int tw = stage ? tx : 16, th = (stage ? ty : 16) * RY;  // back tile in pixels
     for (int bx = 0; bx < (it.Nx + tw - 1) / tw; ++bx)
-      for (int by = 0; by < (it.Ny + th - 1) / th; ++by) sets[kBackward].add(i, bx, by, cb);
+      for (int by = 0; by < (it.Ny + th - 1) / th; ++by) sets[kBackward].add(bx, by);
     const int64_t npix = (int64_t)it.Nx * it.Ny;
-    for (int64_t p = 0; p < (npix + 255) / 256; ++p) sets[kDual].add(i, (int)p, 0, 1.0);
+    sets[kDual].item(1.0);
+    for (int64_t p = 0; p < (npix + 255) / 256; ++p) sets[kDual].add((int)p, 0);
   }
   size_t tiles_at[5];
   std::vector<int4> sorted[5];
@@ -350,7 +380,8 @@ static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_ite
     J.rowY = it.Ny + pad;
     J.sliceX = J.rowX * it.Ny;
     J.sliceY = J.rowY * it.Nx;
-    J.part = nb > kSubBands ? reinterpret_cast<real *>(base + part_at[i]) : nullptr;
+    J.part = bands[i] > kSubBands ? reinterpret_cast<real *>(base + part_at[i]) : nullptr;
+    J.bands = bands[i];
     J.io = order_strides(GT_ORDER_F, it.Nx, it.Ny, 1);
     J.S = reinterpret_cast<const real *>(base + S_at[i]);
     J.tab = reinterpret_cast<const AngleRec<real> *>(base + tab_at[i]);
@@ -411,7 +442,9 @@ static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_ite
   p->n_items = n;
   p->fwd_group = K;
   p->back_rows = RY;
-  p->fwd_bands = nb;
+  p->fwd_banded = bands[0] > 1;
+  p->fwd_partials = partials;
+  p->fwd_bufw = bufw;
   p->fwd_chunk = chunked ? chunk : 1;
   p->back_stage = stage;
   p->back_tile = tx;
@@ -432,35 +465,20 @@ static int plan_create(gt_batch_plan **out, int dtype, int n, const gt_batch_ite
   return GT_OK;
 }
 
-template <typename real, int K, int CH>
-static void launch_fwd_banded(const gt_batch_plan *p, hipStream_t st, const Job<real> *jobs,
-                              dim3 grid, dim3 block) {
-  switch (p->fwd_bands) {
-    case 8:
-      hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, 8>), grid, block, 0, st, jobs,
-                         p->tiles[kForward]);
-      hipLaunchKernelGGL((batch_band_reduce_kernel<real, 8 / kSubBands>), dim3(p->n_tiles[kStage]), dim3(256),
-                         0, st, jobs, p->tiles[kStage]);
-      break;
-    case 4:
-      hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, 4>), grid, block, 0, st, jobs,
-                         p->tiles[kForward]);
-      break;
-    default:
-      hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, 2>), grid, block, 0, st, jobs,
-                         p->tiles[kForward]);
-  }
-}
-
 template <typename real, int K>
 static void launch_fwd_k(const gt_batch_plan *p, hipStream_t st, const Job<real> *jobs, dim3 grid,
                          dim3 block) {
   constexpr int CH = 16 / sizeof(real);
-  if (p->fwd_bands > 1) {
-    if (p->fwd_chunk > 1)
-      launch_fwd_banded<real, K, CH>(p, st, jobs, grid, block);
+  if (p->fwd_banded) {
+    if (p->fwd_bufw)
+      hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, true>), grid, block, 0, st, jobs, p->tiles[kForward]);
+    else if (p->fwd_chunk > 1)
+      hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, CH, false>), grid, block, 0, st, jobs, p->tiles[kForward]);
     else
-      launch_fwd_banded<real, K, 1>(p, st, jobs, grid, block);
+      hipLaunchKernelGGL((batch_fwd_band_kernel<real, K, 1, false>), grid, block, 0, st, jobs, p->tiles[kForward]);
+    if (p->fwd_partials)
+      hipLaunchKernelGGL(batch_band_reduce_kernel<real>, dim3(p->n_tiles[kStage]), dim3(256), 0, st, jobs,
+                         p->tiles[kStage]);
     return;
   }
   if (p->fwd_chunk > 1)
@@ -586,7 +604,7 @@ extern "C" int gt_batch_plan_create(gt_batch_plan **plan, int dtype, int n_items
   t.fwd_group = std::min(t.fwd_group, 16);  // and up to 16 bins per lane
   if (t.automatic) {
     t.fwd_group = 16;
-    t.fwd_bands = 8;
+    t.fwd_bands = 0;  // chosen for each slice
     t.fwd_chunk = 4;
     t.back_rows = 8;
     t.back_stage = 16;

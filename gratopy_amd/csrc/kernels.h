@@ -54,6 +54,7 @@ struct Job {
   const real *imgX, *imgY, *src;
   int64_t rowX, rowY, sliceX, sliceY;
   real *part;  // batched jobs: the slice's band partials of a row-banded forward
+  int bands;   // batched jobs: row bands of the forward
   real *img;
   Strides3 io;
   const real *S;
