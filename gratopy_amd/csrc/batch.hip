@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void batch_relayout_kernel(const Job<real> *__
 // K = 1: tile (slice, bin block, angle block), 64 bins x 4 angles.  K > 1:
 // tile (slice, block of the slice's groups as in the single-problem
 // launches, group_lane).
-template <typename real, int K, int CH = 1>
+template <typename real, int K, int CH = 1, bool BUFW = false>
 __global__ __launch_bounds__(256) void batch_fwd_kernel(const Job<real> *__restrict__ jobs,
                                                         const int4 *__restrict__ tiles) {
   const int4 t = tiles[blockIdx.x];
@@ -118,9 +118,9 @@ __global__ __launch_bounds__(256) void batch_fwd_kernel(const Job<real> *__restr
     if (a >= J.Na) return;
     real *acc = slots + threadIdx.y * 64 + threadIdx.x;
     if (J.fan)
-      fan_fwd_group<real, K, false, CH>(J, g * K, a, 0, acc);
+      fan_fwd_group<real, K, false, CH, BUFW>(J, g * K, a, 0, acc);
     else
-      radon_fwd_group<real, K, false, CH>(J, g * K, a, 0, acc);
+      radon_fwd_group<real, K, false, CH, BUFW>(J, g * K, a, 0, acc);
   }
 }
 
@@ -481,7 +481,9 @@ static void launch_fwd_k(const gt_batch_plan *p, hipStream_t st, const Job<real>
                          p->tiles[kStage]);
     return;
   }
-  if (p->fwd_chunk > 1)
+  if (p->fwd_bufw)
+    hipLaunchKernelGGL((batch_fwd_kernel<real, K, CH, true>), grid, block, 0, st, jobs, p->tiles[kForward]);
+  else if (p->fwd_chunk > 1)
     hipLaunchKernelGGL((batch_fwd_kernel<real, K, CH>), grid, block, 0, st, jobs, p->tiles[kForward]);
   else
     hipLaunchKernelGGL((batch_fwd_kernel<real, K, 1>), grid, block, 0, st, jobs, p->tiles[kForward]);
