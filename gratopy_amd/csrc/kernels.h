@@ -1131,9 +1131,10 @@ constexpr int kStageWidth = 304;
 // (window wider than kStageWidth, or a fan tile reaching t <= 0); its
 // constants give p in padded-sinogram indices (fan: q = ss, k2 = mid_det +
 // 2), clamped to [lo, hi].
+// ty and qy are c1 and k4 times `step`, the distance of a lane's rows.
 template <typename real>
 struct StageWindow {
-  real k0, k1, k2, k3, k4, lo, hi;
+  real k0, k1, k2, k3, k4, ty, qy, lo, hi;
   int w0, n;
 };
 
@@ -1143,7 +1144,7 @@ struct StageWindow {
 // index of margin on each side covers the rounding of the per-pixel evaluation.
 template <typename real, bool FAN>
 __device__ __forceinline__ StageWindow<real> stage_window(const Job<real> &J, int a, int xa, int xb,
-                                                          int ya, int yb) {
+                                                          int ya, int yb, int step) {
   const AngleRec<real> &c = J.tab[a];
   const double mid = FAN ? (double)J.geo[5] + 2.0 : 0.0;
   double pmin = 0, pmax = 0;
@@ -1185,12 +1186,14 @@ __device__ __forceinline__ StageWindow<real> stage_window(const Job<real> &J, in
     W.k0 = (real)(ok ? pc - w0 : pc);
     W.k1 = W.k2 = W.k3 = W.k4 = (real)0;
   }
+  W.ty = c.c[1] * (real)step;
+  W.qy = W.k4 * (real)step;
   W.lo = (real)0.5;
   W.hi = (real)J.Ns + (real)2.5;
   return W;
 }
 
-// Adds one angle's contribution to the RY pixels (xa + dx, ya + dy + r) of
+// Adds one angle's contribution to the RY pixels (xa + dx, ya + dy + step r) of
 // this lane.  STAGED: `row` is the angle's LDS window (no clamp); otherwise
 // the padded sinogram row in memory (clamped as in the unstaged kernel).
 // Row r of the lane is one FMA from row 0, as in back_pixels (row 0 is t0, q0
@@ -1211,12 +1214,12 @@ __device__ __forceinline__ void staged_angle(const AngleRec<real> &c, const Stag
     int ir[RY];
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
-      const real t = FAN ? (r == 0 ? t0 : fma(c.c[1], (real)r, t0)) : (real)1;
-      const real q = r == 0 ? q0 : fma(FAN ? W.k4 : c.c[1], (real)r, q0);
+      const real t = FAN ? (r == 0 ? t0 : fma(W.ty, (real)r, t0)) : (real)1;
+      const real q = r == 0 ? q0 : fma(FAN ? W.qy : c.c[1], (real)r, q0);
       real p = q;
       wr[r] = 1;
       if (FAN) {
-        wr[r] = A::rcp(t);
+        wr[r] = A::rcp_positive(t);  // a staged window has t > 0 on the tile
         p = q * wr[r];
       }
       fr[r] = A::fract(p);
@@ -1237,8 +1240,8 @@ __device__ __forceinline__ void staged_angle(const AngleRec<real> &c, const Stag
   } else {
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
-      const real t = FAN ? (r == 0 ? t0 : fma(c.c[1], (real)r, t0)) : (real)1;
-      const real q = r == 0 ? q0 : fma(FAN ? W.k4 : c.c[1], (real)r, q0);
+      const real t = FAN ? (r == 0 ? t0 : fma(W.ty, (real)r, t0)) : (real)1;
+      const real q = r == 0 ? q0 : fma(FAN ? W.qy : c.c[1], (real)r, q0);
       real p = q, w = 1;
       if (FAN) {
         w = A::rcp(t);
@@ -1283,8 +1286,19 @@ __device__ __forceinline__ void back_staged_tile(const Job<real> &J, int bx, int
   if (a_end < 0) a_end = J.Na;
   constexpr int TY = 256 / TX;  // lane rows
   const int tid = threadIdx.x;
-  const int x = bx * TX + (tid % TX);
-  const int y0 = (by * TY + tid / TX) * RY;
+  // A whole tile of a fan: wave w takes 8 columns and 8 RY rows, a lane every
+  // eighth of them, so that the 64 lanes of one tap read span 8 x 8 pixels: at most
+  // 16 neighbouring bins while a pixel is at most 1.4 bins wide, which LDS serves
+  // without conflicts (rows of 32 pixels have two lanes on a bank in a quarter of
+  // the reads: 2048^2, 1440 angles, 1486 us against 1421; 1024^2, 720 angles, 248
+  // against 214).  Else (a parallel beam, whose rows measure the same: 2048^2 888
+  // against 893; tiles that overhang the image, whose idle rows should not reach far
+  // beyond it): rows of TX lanes with RY consecutive rows each.
+  const bool whole = FAN && (by + 1) * TY * RY <= J.Ny;
+  const int wave = tid >> 6, step = whole ? 8 : 1;
+  const int px = whole ? wave % (TX / 8) * 8 + (tid & 7) : tid % TX;
+  const int py = whole ? wave / (TX / 8) * 8 * RY + (tid >> 3 & 7) : tid / TX * RY;
+  const int x = bx * TX + px, y0 = by * TY * RY + py;
   const bool active = x < J.Nx && y0 < J.Ny;
   const int xa = bx * TX, xb = min(xa + TX - 1, J.Nx - 1);
   // rows evaluated: a lane whose first row is inside the image evaluates all RY
@@ -1292,13 +1306,13 @@ __device__ __forceinline__ void back_staged_tile(const Job<real> &J, int bx, int
   const int Nsp = J.Ns + 4;
   const real *Sz = J.S + (int64_t)z * J.Na * Nsp;
   // the lane's first pixel relative to the tile corner (xa, ya)
-  const real dx = (real)(tid % TX), dy = (real)((tid / TX) * RY);
+  const real dx = (real)px, dy = (real)py;
   real acc[RY];
 #pragma unroll
   for (int r = 0; r < RY; ++r) acc[r] = 0;
   for (int a0 = a_begin; a0 < a_end; a0 += CA) {
     const int na = min(CA, a_end - a0);
-    if (tid < na) win[tid] = stage_window<real, FAN>(J, a0 + tid, xa, xb, ya, yb);
+    if (tid < na) win[tid] = stage_window<real, FAN>(J, a0 + tid, xa, xb, ya, yb, step);
     __syncthreads();
     // every angle of the chunk staged (a wave-uniform vote): the accumulation
     // loop below then runs without the per-angle branch to the memory path
@@ -1370,7 +1384,7 @@ __device__ __forceinline__ void back_staged_tile(const Job<real> &J, int bx, int
   if (!active) return;
 #pragma unroll
   for (int r = 0; r < RY; ++r) {
-    const int y = y0 + r;
+    const int y = y0 + step * r;
     if (y >= J.Ny) break;
     if (part)
       part[(((int64_t)band * J.Nz + z) * J.Ny + y) * J.Nx + x] = acc[r];
