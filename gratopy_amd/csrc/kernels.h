@@ -712,7 +712,8 @@ __device__ __forceinline__ void fan_fwd_group(const Job<real> &J, int s0, int a,
     auto chunk = [&](const RowChunk<real, CH> &c) {
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
-        const real r = A::rcp(i == 0 ? t : t + ts[i]);
+        // positive within the strip; elsewhere anything (NaN too) is discarded
+        const real r = A::rcp_positive(i == 0 ? t : t + ts[i]);
         const real p = A::clamp((i == 0 ? q : q + qs[i]) * r, lo, hi);
         deposit(acc, p, c.v[i] * r);
       }
