@@ -422,7 +422,9 @@ def roofline(workload, direction, seconds, work, elem=4):
 
 
 def launch_shapes(lib, fan, N, Ns, Na, Nz):
-    """The launch shapes the library takes for the stack (gt_projection_shape)."""
+    """The general launch shapes for the stack (gt_projection_shape).  Automatic
+    calls on stacks of slices run the slice-batched kernels instead, explicit
+    variants run these."""
     import ctypes
 
     out = {}

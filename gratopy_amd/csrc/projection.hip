@@ -741,11 +741,12 @@ static int check_sizes(const Layout &L) {
 
 static size_t elem_size(int dtype) { return dtype == GT_FLOAT64 ? 8 : 4; }
 
-// Launch shape of one call: the tuning knobs, or (GT_TUNE_AUTO, the default)
-// a choice by the geometry and the work of the call, Nx*Ny*Na*Nz pixel-angles,
-// from autotuner trials on MI355X (256^2 to 32 x 2048^2, parallel and fan
-// beam): small problems need row or angle bands to fill the GPU; larger ones
-// run the chunked forward and the LDS-staged backprojection.
+// General launch shape of one call: the tuning knobs, or (GT_TUNE_AUTO, the
+// default, where no route of its own below applies or its workspace is missing) a
+// choice by the geometry and the work of the call, Nx*Ny*Na*Nz pixel-angles, from
+// autotuner trials on MI355X (256^2 to 32 x 2048^2, parallel and fan beam): small
+// problems need row or angle bands to fill the GPU; larger ones run the chunked
+// forward and the LDS-staged backprojection.
 struct FwdShape {
   int K, bands, chunk;  // bands and chunked reads need bin groups (K > 1)
   bool compact;         // banded: launch only the groups that meet each band (FwdPlan)
@@ -850,7 +851,7 @@ static bool back_is_small(int dtype, const Layout &L) {
 //   parallel 512^2, 360 angles   8: - / 70.0 / 69.2 / 70.5, 16: 80.3 / 75.5 / 74.8 / 73.3  (70.1)
 //   parallel 1024^2, 720 angles  8: 369 / 355 / 353 / 358, 16: 375 / 350 / 332 / 341  (354)
 //   fan 1024^2, 720 angles       8: 412 / 416 / 411 / -, 16: 365 / 346 / 336 / 360  (415)
-//   parallel 2048^2, 1440 angles 16: 2321 / 2204 / 2211 / 2194  (2307)
+//   parallel 2048^2, 1440 angles 16: 2321 / 2204 / 2211 / 2194  (2307; 2095 with walk_chunks)
 //   fan 2048^2, 1440 angles      16: 2282 / 2223 / 2167 / 2376  (2491)
 // 48 bands of fewer than 10 rows lose to 32, and launches that fill the GPU many
 // times over take 16, for the memory of the sums.  16 bins a lane need enough lanes:

@@ -95,17 +95,20 @@ int gt_tune_get(int key);
  * truncated to n bytes); returns the full message length. */
 size_t gt_last_error(char *buf, size_t n);
 
-/* Workspace bytes needed by gt_{radon,fan}_{fwd,back} for these sizes.
+/* Workspace bytes that gt_{radon,fan}_{fwd,back} take for these sizes.
  * geometry is that of the call (GT_GEOMETRY_RADON or GT_GEOMETRY_FAN: the
  * automatic launch shape, and with it the workspace, depends on it);
  * adjoint = 0 for the forward projection, 1 for the backprojection;
- * in_order is the order of the input array of that call.  A call given less
- * workspace than it needs returns GT_ENOSPC. */
+ * in_order is the order of the input array of that call.  Automatic calls given
+ * less run the general launch shape (gt_projection_shape) where that fits, with
+ * results equal to rounding; below its needs a call returns GT_ENOSPC. */
 size_t gt_projection_workspace_bytes(int geometry, int adjoint, int dtype, int Nx, int Ny,
                                      int Ns, int Na, int Nz, int in_order);
 
-/* The launch shape a projection call with these sizes takes under the current
- * knobs (the automatic choice when GT_TUNE_AUTO = 1): forward: shape[0..3] =
+/* The general launch shape of a projection call with these sizes under the current
+ * knobs (the automatic choice when GT_TUNE_AUTO = 1; automatic calls leave it for
+ * kernels of their own on stacks of slices, for small calls, and for more row bands
+ * on single slices): forward: shape[0..3] =
  * detector bins per lane, row bands, pixels per strip load, compacted (0/1);
  * backprojection: shape[0..3] = pixels per lane, angle bands, angles per LDS
  * staging chunk (0 = unstaged), staged tile width.  No reference counterpart
@@ -149,10 +152,10 @@ int gt_fan_back(gt_stream_t stream, int dtype, void *img, const void *sino, cons
  * counterpart in the reference: for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
  * Allocates nothing.  The stream must belong to the current device.  A call whose
- * workspace (gt_projection_workspace_bytes) exceeds the array returns GT_ENOSPC.
+ * general launch shape needs more than the array returns GT_ENOSPC.
  * Every call on one GPU uses the same array: calls that overlap on one GPU (on
  * different streams, or from different threads) race.  Results are those of the
- * entry points above. */
+ * entry points above with that much workspace. */
 #define GT_NOALLOC_SCRATCH_BYTES ((size_t)128 << 20)
 int gt_projection_noalloc(gt_stream_t stream, int geometry, int adjoint, int dtype, void *out,
                           const void *in, const void *ofs, const void *sdpd, const void *geo,
