@@ -930,7 +930,7 @@ static size_t back_stack_ws(int dtype, const Layout &L, const BackStackShape &s)
 
 static size_t back_need(int dtype, const Layout &L) {
   const BackStackShape s = back_stack_shape(dtype, L);
-  return s.g ? back_stack_ws(dtype, L, s) : back_ws(dtype, L);
+  return s.g ? std::max(back_ws(dtype, L), back_stack_ws(dtype, L, s)) : back_ws(dtype, L);
 }
 
 // Slice-batched forward: g slice groups per lane, halves x 64 rays per block,
@@ -986,8 +986,8 @@ static size_t fwd_stack_ws(int dtype, const Layout &L, const FwdStackShape &s) {
 
 static size_t fwd_need(int dtype, const Layout &L, int img_order) {
   const FwdStackShape s = fwd_stack_shape(dtype, L);
-  if (s.g) return fwd_stack_ws(dtype, L, s);
   const size_t need = fwd_ws(dtype, L, img_order);
+  if (s.g) return std::max(need, fwd_stack_ws(dtype, L, s));
   return tuning().automatic && !fwd_is_small(L) ? std::max(need, fwd_run_ws(dtype, L)) : need;
 }
 
@@ -1105,13 +1105,13 @@ static int fwd_impl(hipStream_t st, real *sino, const real *img, const real *ofs
                     const real *sdpd, const real *geo, const Layout &L, int sino_order,
                     int img_order, void *ws, size_t ws_bytes) {
   const int dtype = sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32;
+  size_t need = fwd_ws(dtype, L, img_order);
+  if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
+  GT_REQUIRE(need == 0 || ws != nullptr, "workspace pointer is NULL");
   const FwdStackShape ss = fwd_stack_shape(dtype, L);
   if (ss.g && ws != nullptr && ws_bytes >= fwd_stack_ws(dtype, L, ss))
     return fwd_stack_impl<real, FAN>(st, sino, img, ofs, sdpd, geo, L, sino_order, img_order,
                                      static_cast<char *>(ws), ss);
-  size_t need = fwd_ws(dtype, L, img_order);
-  if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
-  GT_REQUIRE(need == 0 || ws != nullptr, "workspace pointer is NULL");
   const Strides3 is = order_strides(img_order, L.Nx, L.Ny, L.Nz);
   char *w = static_cast<char *>(ws);
   Job<real> J = make_job<real>(FAN, L, ofs, sdpd, geo);
@@ -1266,13 +1266,13 @@ static int back_impl(hipStream_t st, real *img, const real *sino, const real *of
                      const real *sdpd, const real *geo, const Layout &L, int img_order,
                      int sino_order, void *ws, size_t ws_bytes) {
   const int dtype = sizeof(real) == 8 ? GT_FLOAT64 : GT_FLOAT32;
+  const size_t need = back_ws(dtype, L);
+  if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
+  GT_REQUIRE(ws != nullptr, "workspace pointer is NULL");
   const BackStackShape ss = back_stack_shape(dtype, L);
   if (ss.g && ws != nullptr && ws_bytes >= back_stack_ws(dtype, L, ss))
     return back_stack_impl<real, FAN>(st, img, sino, ofs, sdpd, geo, L, img_order, sino_order,
                                       static_cast<char *>(ws), ss);
-  const size_t need = back_ws(dtype, L);
-  if (ws_bytes < need) return fail(GT_ENOSPC, "projection workspace too small");
-  GT_REQUIRE(ws != nullptr, "workspace pointer is NULL");
   if (back_is_small(dtype, L)) {
     Job<real> J = make_job<real>(FAN, L, ofs, sdpd, geo);
     J.img = img;
